@@ -25,6 +25,12 @@
 #include "hooks.hpp"
 #include <type_traits>
 
+// One object per population storage, compiled side by side (LBM3_STEP_STORE:
+// the LBM3_STORE_* code of this object's storage; undefined: all of them in
+// one object).  What does not depend on the storage is defined in each and
+// merged by the linker; its kernels are local to their object.
+#define LBM3_SHARED_DEF __attribute__((weak))
+
 namespace lbm3 {
 
 template <class S, bool FLIP>
@@ -469,7 +475,7 @@ __global__ __launch_bounds__(256) void k_open_groups(StepArgs<S> a)
 }
 
 // the plain fluid cells of the open groups: record -5 in place of -1 / -2
-__global__ __launch_bounds__(256) void k_mark_groups(const int *groups, int count, int G, int N, int2 *cellRow)
+static __global__ __launch_bounds__(256) void k_mark_groups(const int *groups, int count, int G, int N, int2 *cellRow)
 {
     const long long t = blockIdx.x * 256LL + threadIdx.x;
     if (t >= (long long)count * G) return;
@@ -483,7 +489,7 @@ __global__ __launch_bounds__(256) void k_mark_groups(const int *groups, int coun
 // it skips (record >= 0 or <= -3, and the padding past N), per 256 cells the
 // row of the first one; with `open` non-null the open cells (record <= -8) are
 // the bulk kernel's too, marked in `open`
-__global__ __launch_bounds__(256) void k_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *tileRow,
+static __global__ __launch_bounds__(256) void k_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *tileRow,
                                                    uint64_t *open, uint64_t *rotor)
 {
     const int cell = blockIdx.x * 256 + threadIdx.x;
@@ -505,7 +511,7 @@ __global__ __launch_bounds__(256) void k_bulk_mask(const int2 *cellRow, int N, u
     if (threadIdx.x == 0) tileRow[blockIdx.x] = row;
 }
 
-void launch_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *tileRow, uint64_t *open, uint64_t *rotor,
+LBM3_SHARED_DEF void launch_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *tileRow, uint64_t *open, uint64_t *rotor,
                       hipStream_t s)
 {
     if (N <= 0) return;
@@ -514,7 +520,7 @@ void launch_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *tileRow, 
 
 // the cells of the open groups leave the bulk kernel's view: skip bits set,
 // open bits cleared (a group of 8 or 16 aligned cells lies in one 64-bit word)
-__global__ __launch_bounds__(256) void k_group_bits(const int *groups, int count, int G, uint64_t *skip, uint64_t *open)
+static __global__ __launch_bounds__(256) void k_group_bits(const int *groups, int count, int G, uint64_t *skip, uint64_t *open)
 {
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (t >= count) return;
@@ -524,13 +530,13 @@ __global__ __launch_bounds__(256) void k_group_bits(const int *groups, int count
     atomicAnd(reinterpret_cast<unsigned long long *>(open + (first >> 6)), ~bits);
 }
 
-void launch_group_bits(const int *groups, int count, int G, uint64_t *skip, uint64_t *open, hipStream_t s)
+LBM3_SHARED_DEF void launch_group_bits(const int *groups, int count, int G, uint64_t *skip, uint64_t *open, hipStream_t s)
 {
     if (count <= 0) return;
     k_group_bits<<<(count + 255) / 256, 256, 0, s>>>(groups, count, G, skip, open);
 }
 
-void launch_mark_groups(const int *groups, int count, int G, int N, int2 *cellRow, hipStream_t s)
+LBM3_SHARED_DEF void launch_mark_groups(const int *groups, int count, int G, int N, int2 *cellRow, hipStream_t s)
 {
     if (count <= 0) return;
     hipLaunchKernelGGL(k_mark_groups, dim3((unsigned)(((long long)count * G + 255) / 256)), dim3(256), 0, s, groups, count,
@@ -634,7 +640,7 @@ __device__ __forceinline__ void wall_cell(const StepArgs<S> &a, int wm)
 }
 
 // neighbour cells of every open-boundary cell, decoded once at setup
-__global__ __launch_bounds__(256) void k_open_nb(Topology t, int count, const int *cell, int4 *out)
+static __global__ __launch_bounds__(256) void k_open_nb(Topology t, int count, const int *cell, int4 *out)
 {
     const int x = blockIdx.x * 256 + threadIdx.x;
     if (x >= count) return;
@@ -708,7 +714,7 @@ __global__ __launch_bounds__(256, walls_waves<S>(OPEN)) void k_collide_stream_wa
 // with rotorCand, the fluid cells the rotors can reach get -4, and with openOf
 // the open-boundary cells get -(8 + open-list index), in place of
 // their wall-map code (they are never wall-adjacent when this is used)
-__global__ __launch_bounds__(256) void k_fast_topo(Topology t, const int *wallMap, const int *openOf, const uint8_t *rotorCand,
+static __global__ __launch_bounds__(256) void k_fast_topo(Topology t, const int *wallMap, const int *openOf, const uint8_t *rotorCand,
                                                    int2 *cellRow, int4 *rows)
 {
     const int cell = blockIdx.x * 256 + threadIdx.x;
@@ -724,7 +730,7 @@ __global__ __launch_bounds__(256) void k_fast_topo(Topology t, const int *wallMa
 
 // cells a later pass of the step reads or writes as a whole (periodic copies,
 // interface stencils) must not carry a boundary condition that is still pending
-__global__ __launch_bounds__(256) void k_open_conflicts(const int *cells, int count, int mode, const int *openOf,
+static __global__ __launch_bounds__(256) void k_open_conflicts(const int *cells, int count, int mode, const int *openOf,
                                                         const int *wallMap, const uint8_t *cand, FastTopo t, int *flag)
 {
     const int x = blockIdx.x * 256 + threadIdx.x;
@@ -744,7 +750,7 @@ __global__ __launch_bounds__(256) void k_open_conflicts(const int *cells, int co
 
 // cells a rotor can reach at some angle: within its bounds' distance from the
 // axis (plus two level spacings) and inside its axial extent (the same margin)
-__global__ __launch_bounds__(256) void k_rotor_reach(Topology t, LevelGeom g, RotorReachSet R, uint8_t *cand)
+static __global__ __launch_bounds__(256) void k_rotor_reach(Topology t, LevelGeom g, RotorReachSet R, uint8_t *cand)
 {
     const int cell = blockIdx.x * 256 + threadIdx.x;
     if (cell >= t.N) return;
@@ -774,13 +780,13 @@ __global__ __launch_bounds__(256) void k_rotor_reach(Topology t, LevelGeom g, Ro
     cand[cell] = hit;
 }
 
-void launch_rotor_reach(const Topology &t, const LevelGeom &g, const RotorReachSet &R, uint8_t *cand, hipStream_t s)
+LBM3_SHARED_DEF void launch_rotor_reach(const Topology &t, const LevelGeom &g, const RotorReachSet &R, uint8_t *cand, hipStream_t s)
 {
     if (t.N <= 0) return;
     hipLaunchKernelGGL(k_rotor_reach, dim3((unsigned)((t.N + 255) / 256)), dim3(256), 0, s, t, g, R, cand);
 }
 
-__global__ __launch_bounds__(256) void k_scatter_index(const int *cell, int count, int *openOf)
+static __global__ __launch_bounds__(256) void k_scatter_index(const int *cell, int count, int *openOf)
 {
     const int x = blockIdx.x * 256 + threadIdx.x;
     if (x < count) openOf[cell[x]] = x;
@@ -964,7 +970,7 @@ __global__ __launch_bounds__(256) void k_cell_sums(const S *f, Topology topo, co
 
 // one block: out = sum of partial[0..n) / divisor, added to the value out holds
 // when accumulate is set (levels weighted and summed on the device, in order)
-__global__ __launch_bounds__(256) void k_sum_partials(const double *partial, int n, double *out, double divisor, int accumulate)
+static __global__ __launch_bounds__(256) void k_sum_partials(const double *partial, int n, double *out, double divisor, int accumulate)
 {
     __shared__ double lds[4];
     double v = 0.0;
@@ -978,7 +984,7 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double *partial, int
 // uNormal, rho uNormal, rho uNormal |uNormal|, dRho, dRho uNormal,
 // rho uNormal^3 / 2 (time averages of the accumulators, lattice units) and the
 // tracked-entry count; partial[block * 7 + k]
-__global__ __launch_bounds__(256) void k_open_stats(const double *dRhoCum, const double *uNormalCum, const uint32_t *meta,
+static __global__ __launch_bounds__(256) void k_open_stats(const double *dRhoCum, const double *uNormalCum, const uint32_t *meta,
                                                     int start, int count, double invSpan, double *partial)
 {
     __shared__ double lds[7 * 4];
@@ -1002,7 +1008,7 @@ __global__ __launch_bounds__(256) void k_open_stats(const double *dRhoCum, const
     }
 }
 
-int launch_open_stats(const double *dRhoCum, const double *uNormalCum, const uint32_t *meta, int start, int count,
+LBM3_SHARED_DEF int launch_open_stats(const double *dRhoCum, const double *uNormalCum, const uint32_t *meta, int start, int count,
                       double invSpan, double *partial, hipStream_t s)
 {
     const int blocks = (count + 255) / 256;
@@ -1012,7 +1018,7 @@ int launch_open_stats(const double *dRhoCum, const double *uNormalCum, const uin
 
 // per-wall-body sums of the accumulated force and its torque about `origin`;
 // out[body*6 + {Fx,Fy,Fz,Tx,Ty,Tz}] per block
-__global__ __launch_bounds__(256) void k_wall_force(const double *gWall, int W, const uint32_t *wallData, const int *wallIndex,
+static __global__ __launch_bounds__(256) void k_wall_force(const double *gWall, int W, const uint32_t *wallData, const int *wallIndex,
                                                     Topology topo, LevelGeom g, double ox, double oy, double oz, int nBodies,
                                                     double *partial)
 {
@@ -1250,7 +1256,7 @@ void launch_open_cells(const StepArgs<S> &a, bool flip, hipStream_t s)
 
 // velocity profile factor of each open-list entry: its rule's radial profile
 // at the cell centre (getOpenBC of the pipe cases, poiseuilleFlowMain.cu:58-75)
-__global__ __launch_bounds__(256) void k_open_scale(Topology t, LevelGeom g, int count, const int *cell,
+static __global__ __launch_bounds__(256) void k_open_scale(Topology t, LevelGeom g, int count, const int *cell,
                                                      const uint32_t *meta, OpenProfiles P, float *scale)
 {
     const int x = blockIdx.x * 256 + threadIdx.x;
@@ -1262,27 +1268,27 @@ __global__ __launch_bounds__(256) void k_open_scale(Topology t, LevelGeom g, int
     scale[x] = profile_factor(P.p[open_meta_record(meta[x])], px, py, pz);
 }
 
-void launch_open_scale(const Topology &t, const LevelGeom &g, int count, const int *cell, const uint32_t *meta,
+LBM3_SHARED_DEF void launch_open_scale(const Topology &t, const LevelGeom &g, int count, const int *cell, const uint32_t *meta,
                        const OpenProfiles &P, float *scale, hipStream_t s)
 {
     if (count <= 0) return;
     k_open_scale<<<(count + 255) / 256, 256, 0, s>>>(t, g, count, cell, meta, P, scale);
 }
 
-void launch_open_nb(const Topology &t, int count, const int *cell, int4 *out, hipStream_t s)
+LBM3_SHARED_DEF void launch_open_nb(const Topology &t, int count, const int *cell, int4 *out, hipStream_t s)
 {
     if (count <= 0) return;
     hipLaunchKernelGGL(k_open_nb, dim3(blocks_for(count)), dim3(256), 0, s, t, count, cell, out);
 }
 
-void launch_fast_topo(const Topology &t, const int *wallMap, const int *openOf, const uint8_t *rotorCand, int2 *cellRow,
+LBM3_SHARED_DEF void launch_fast_topo(const Topology &t, const int *wallMap, const int *openOf, const uint8_t *rotorCand, int2 *cellRow,
                       int4 *rows, hipStream_t s)
 {
     if (t.N <= 0) return;
     hipLaunchKernelGGL(k_fast_topo, dim3(blocks_for(t.N)), dim3(256), 0, s, t, wallMap, openOf, rotorCand, cellRow, rows);
 }
 
-void launch_open_conflicts(const int *cells, int count, int mode, const int *openOf, const int *wallMap,
+LBM3_SHARED_DEF void launch_open_conflicts(const int *cells, int count, int mode, const int *openOf, const int *wallMap,
                            const uint8_t *cand, const FastTopo &t, int *flag, hipStream_t s)
 {
     if (count <= 0) return;
@@ -1290,20 +1296,20 @@ void launch_open_conflicts(const int *cells, int count, int mode, const int *ope
                        t, flag);
 }
 
-void launch_scatter_index(const int *cell, int count, int *openOf, hipStream_t s)
+LBM3_SHARED_DEF void launch_scatter_index(const int *cell, int count, int *openOf, hipStream_t s)
 {
     if (count <= 0) return;
     hipLaunchKernelGGL(k_scatter_index, dim3(blocks_for(count)), dim3(256), 0, s, cell, count, openOf);
 }
 
 // openOf[cell of entry] = entry, for the listed open-list entries only
-__global__ __launch_bounds__(256) void k_scatter_entries(const int *cell, const int *list, int count, int *openOf)
+static __global__ __launch_bounds__(256) void k_scatter_entries(const int *cell, const int *list, int count, int *openOf)
 {
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (t < count) openOf[cell[list[t]]] = list[t];
 }
 
-void launch_scatter_entries(const int *cell, const int *list, int count, int *openOf, hipStream_t s)
+LBM3_SHARED_DEF void launch_scatter_entries(const int *cell, const int *list, int count, int *openOf, hipStream_t s)
 {
     if (count <= 0) return;
     hipLaunchKernelGGL(k_scatter_entries, dim3(blocks_for(count)), dim3(256), 0, s, cell, list, count, openOf);
@@ -1373,7 +1379,7 @@ int launch_mass(const S *f, const Topology &t, const int *wallMap, const uint32_
     return (int)nb;
 }
 
-void launch_wall_force(const double *gWall, int W, const uint32_t *wallData, const int *wallIndex, const Topology &t,
+LBM3_SHARED_DEF void launch_wall_force(const double *gWall, int W, const uint32_t *wallData, const int *wallIndex, const Topology &t,
                        const LevelGeom &g, const double origin[3], int nBodies, double *partial, hipStream_t s)
 {
     if (W <= 0) return;
@@ -1404,7 +1410,7 @@ void launch_multi_step(const MultiDesc<S> *D, const int *starts, int n, const in
 
 // image of the section: per pixel {dRho, ux, uy, uz, marker, gridID} before
 // conversion; marker 1 (solid) and zeros where no level writes
-__global__ __launch_bounds__(256) void k_cut_clear(float *img, long long pixels)
+static __global__ __launch_bounds__(256) void k_cut_clear(float *img, long long pixels)
 {
     const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
     if (p >= pixels) return;
@@ -1477,7 +1483,7 @@ __global__ __launch_bounds__(256) void k_section_cut(const S *f, Topology topo, 
 
 // physical units and the plane's velocity order, per pixel (:296-329):
 // {p [Pa], u horizontal, u vertical, u normal [m/s], marker, res [mm]}
-__global__ __launch_bounds__(256) void k_cut_finish(float *img, long long pixels, CutUnits u)
+static __global__ __launch_bounds__(256) void k_cut_finish(float *img, long long pixels, CutUnits u)
 {
     const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
     if (p >= pixels) return;
@@ -1545,12 +1551,12 @@ template <class S> void launch_section_cut(const S *f, const Topology &t, const 
     else k_section_cut<S, false><<<g, 256, 0, s>>>(f, t, wallMap, cd, d, img);
 }
 
-void launch_cut_clear(float *img, long long pixels, hipStream_t s)
+LBM3_SHARED_DEF void launch_cut_clear(float *img, long long pixels, hipStream_t s)
 {
     if (pixels > 0) k_cut_clear<<<(unsigned)((pixels + 255) / 256), 256, 0, s>>>(img, pixels);
 }
 
-void launch_cut_finish(float *img, long long pixels, const CutUnits &u, hipStream_t s)
+LBM3_SHARED_DEF void launch_cut_finish(float *img, long long pixels, const CutUnits &u, hipStream_t s)
 {
     if (pixels > 0) k_cut_finish<<<(unsigned)((pixels + 255) / 256), 256, 0, s>>>(img, pixels, u);
 }
@@ -1576,13 +1582,27 @@ void launch_cut_finish(float *img, long long pixels, const CutUnits &u, hipStrea
                                           double *, const Codec &, bool, hipStream_t, double, bool);              \
     template int launch_mass<S>(const S *, const Topology &, const int *, const uint32_t *, double *, double *,       \
                                 const Codec &, bool, hipStream_t, double, bool);
+#ifndef LBM3_STEP_STORE
+#define LBM3_STEP_STORE -1
+#endif
+#define LBM3_STEP_HAS(store) (LBM3_STEP_STORE == -1 || LBM3_STEP_STORE == store)
+#if LBM3_STEP_HAS(LBM3_STORE_F32)
 LBM3_INSTANTIATE(float)
-LBM3_INSTANTIATE(double)
-LBM3_INSTANTIATE(__half)
-LBM3_INSTANTIATE(__hip_bfloat16)
-LBM3_INSTANTIATE(f16c)
 template void launch_collide_batch<float>(float *, int, const Relax<float> &, hipStream_t);
+#endif
+#if LBM3_STEP_HAS(LBM3_STORE_F64)
+LBM3_INSTANTIATE(double)
 template void launch_collide_batch<double>(double *, int, const Relax<double> &, hipStream_t);
+#endif
+#if LBM3_STEP_HAS(LBM3_STORE_F16)
+LBM3_INSTANTIATE(__half)
+#endif
+#if LBM3_STEP_HAS(LBM3_STORE_BF16)
+LBM3_INSTANTIATE(__hip_bfloat16)
+#endif
+#if LBM3_STEP_HAS(LBM3_STORE_F16C)
+LBM3_INSTANTIATE(f16c)
+#endif
 
 } // namespace lbm3
 
@@ -1591,7 +1611,7 @@ template void launch_collide_batch<double>(double *, int, const Relax<double> &,
 // ---------------------------------------------------------------------------
 namespace lbm3 {
 typedef float f4v __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void k_copy(const float4 *__restrict__ a4, float4 *__restrict__ b4, long long n4,
+static __global__ __launch_bounds__(256) void k_copy(const float4 *__restrict__ a4, float4 *__restrict__ b4, long long n4,
                                               const float *__restrict__ at, float *__restrict__ bt, int tail)
 {
     // four independent 16-byte loads in flight per thread before the stores,
@@ -1623,7 +1643,7 @@ template <class E> __global__ __launch_bounds__(256) void k_relayout(const E *sr
     else dst[pop_index(q, c)] = src[x];
 }
 
-void launch_relayout(const void *src, void *dst, int N, int elemBytes, bool toPlanes, hipStream_t s)
+LBM3_SHARED_DEF void launch_relayout(const void *src, void *dst, int N, int elemBytes, bool toPlanes, hipStream_t s)
 {
     if (N <= 0) return;
     const unsigned g = blocks_for(27LL * N);
@@ -1632,7 +1652,7 @@ void launch_relayout(const void *src, void *dst, int N, int elemBytes, bool toPl
     else hipLaunchKernelGGL(k_relayout<uint64_t>, dim3(g), dim3(256), 0, s, (const uint64_t *)src, (uint64_t *)dst, N, int(toPlanes));
 }
 
-void launch_copy(const void *a, void *b, long long bytes, hipStream_t s)
+LBM3_SHARED_DEF void launch_copy(const void *a, void *b, long long bytes, hipStream_t s)
 {
     const long long n4 = bytes / 16;
     const int tail = (int)((bytes - 16 * n4) / 4);
