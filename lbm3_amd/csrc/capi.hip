@@ -71,11 +71,11 @@ template <class T> static int upload(DBuf<T> &b, const T *host, long long n, hip
 static int refresh_bulk_mask(Sim &s, Level &l)
 {
     const long long blocks = (l.N + 255) / 256;
-    if (l.tileRow.n < blocks) HIPCHK(l.tileRow.alloc(blocks > 0 ? blocks : 1));
+    if (l.waveRow.n < 4 * blocks) HIPCHK(l.waveRow.alloc(blocks > 0 ? 4 * blocks : 4));
     if (l.bulkSkip.n < 4 * blocks) HIPCHK(l.bulkSkip.alloc(blocks > 0 ? 4 * blocks : 4));
     if (l.openInBulk && l.openBits.n < 4 * blocks) HIPCHK(l.openBits.alloc(blocks > 0 ? 4 * blocks : 4));
     if (l.rotorInBulk && l.rotorBits.n < 4 * blocks) HIPCHK(l.rotorBits.alloc(blocks > 0 ? 4 * blocks : 4));
-    launch_bulk_mask(l.cellRow.p, l.N, l.bulkSkip.p, l.tileRow.p, l.openInBulk ? l.openBits.p : nullptr,
+    launch_bulk_mask(l.cellRow.p, l.N, l.bulkSkip.p, l.waveRow.p, l.openInBulk ? l.openBits.p : nullptr,
                      l.rotorInBulk ? l.rotorBits.p : nullptr, s.stream);
     return check_hip(hipGetLastError(), "bulk mask");
 }
@@ -135,8 +135,8 @@ int finish_level_setup(Sim &s, int level)
     if (l.N > (1LL << 31) - 1 - LBM3_TILE) return set_error(LBM3_E_MEMORY, "a level exceeds 2^31 cells");
     if (const int rc = setup_local_bc(s, level)) return rc;
     HIPCHK(l.cellRow.alloc(l.N > 0 ? l.N : 1));
-    HIPCHK(l.rowTab.alloc(l.nRows > 0 ? l.nRows : 1));
-    launch_fast_topo(topo_of(l), l.wallMap.p, nullptr, nullptr, l.cellRow.p, l.rowTab.p, s.stream);
+    HIPCHK(l.rowTab.alloc(l.nRows + kRowPad));
+    launch_fast_topo(topo_of(l), l.nRows, l.wallMap.p, nullptr, nullptr, l.cellRow.p, l.rowTab.p, s.stream);
     if (const int rc = refresh_bulk_mask(s, l)) return rc;
     // interface neighbour tables that read this level are derived again
     l.F2C.nbReady = l.C2F.nbReady = false;
@@ -145,6 +145,8 @@ int finish_level_setup(Sim &s, int level)
     l.rotorDev.release();
     l.rotorCellCount = 0;
     l.openFusionChecked = false;
+    l.imagesReady = false;
+    l.ghostsStale = false;
     l.fusedOpen = false;
     l.openInBulk = false;
     l.rotorInBulk = false;
@@ -186,6 +188,43 @@ static bool wide_of(const Sim &s, const Level &l)
     return 27LL * padded_cells(l.N) * (long long)storage_bytes(s.storage) > 0xFFFFFFFFLL;
 }
 
+// Whether the bulk kernel can step the periodic ghosts from their source cells
+// (one launch per step instead of a copy after each): a single level that is a
+// full box of plain fluid cells where ghosts and sources lie.  Levels with
+// wall-adjacent or rotor cells, whose kernels could step a ghost, an interface
+// that reads ghosts, or 64-bit offsets keep the copy.
+static int prepare_images(Sim &s, Level &l)
+{
+    l.imagesReady = false;
+    const long long box = (long long)l.info.cellCountX * l.info.cellCountY * l.info.cellCountZ;
+    if (l.nPeriodic == 0 || s.levels != 1 || l.W > 0 || !l.rotors.empty() || l.laneRot || l.N != box || wide_of(s, l)) return 0;
+    const long long words = 4 * ((l.N + 255) / 256);
+    DBuf<int> flag;
+    HIPCHK(flag.alloc(1));
+    HIPCHK(l.ghostSkip.alloc(words));
+    HIPCHK(l.imageSources.alloc(words));
+    HIPCHK(l.imageHead.alloc(l.N));
+    HIPCHK(l.imageInfo.alloc(l.nPeriodic));
+    HIPCHK(l.imageNb.alloc(2LL * l.nPeriodic));
+    HIPCHK(hipMemsetAsync(flag.p, 0, sizeof(int), s.stream));
+    HIPCHK(hipMemsetAsync(l.imageSources.p, 0, sizeof(uint64_t) * (size_t)words, s.stream));
+    HIPCHK(hipMemcpyAsync(l.ghostSkip.p, l.bulkSkip.p, sizeof(uint64_t) * (size_t)words, hipMemcpyDeviceToDevice, s.stream));
+    FastTopo ft{};
+    ft.N = l.N;
+    ft.cellRow = l.cellRow.p;
+    ft.rows = l.rowTab.p;
+    ft.skip = l.bulkSkip.p;
+    ft.nRows = l.nRows;
+    launch_images(topo_of(l), ft, l.geom, l.nPeriodic, l.perIndex.p, l.perSource.p, l.ghostSkip.p, l.imageSources.p,
+                  l.imageHead.p, l.imageInfo.p, l.imageNb.p, flag.p, s.stream);
+    HIPCHK(hipGetLastError());
+    int bad = 0;
+    HIPCHK(hipMemcpyAsync(&bad, flag.p, sizeof(int), hipMemcpyDeviceToHost, s.stream));
+    HIPCHK(hipStreamSynchronize(s.stream));
+    l.imagesReady = bad == 0;
+    return 0;
+}
+
 // Decide which special cells of level L get kernels of their own and rebuild
 // the per-cell records the bulk kernel skips them by:
 // * the cells a rotor can reach at some angle (record -4, k_rotor_cells);
@@ -199,6 +238,7 @@ static int prepare_open_fusion(Sim &s, int L)
     Level &l = s.L[L];
     if (const int rc = settle_open(s, L)) return rc;   // a condition pending under the old records
     l.openFusionChecked = true;
+    l.imagesReady = false;
     l.fusedOpen = false;
     l.openInBulk = false;
     l.laneRot = false;
@@ -268,7 +308,7 @@ static int prepare_open_fusion(Sim &s, int L)
             launch_scatter_entries(l.openCell.p, l.fusedEntries.p, l.nFusedEntries, openOf.p, s.stream);
         }
     }
-    launch_fast_topo(topo_of(l), l.wallMap.p, fuse ? openOf.p : nullptr, cand, l.cellRow.p, l.rowTab.p, s.stream);
+    launch_fast_topo(topo_of(l), l.nRows, l.wallMap.p, fuse ? openOf.p : nullptr, cand, l.cellRow.p, l.rowTab.p, s.stream);
     HIPCHK(hipGetLastError());
     l.nOpenGroups = 0;
     // the rotor cells in the bulk kernel (the kernel takes open cells or rotor
@@ -337,7 +377,7 @@ static int prepare_open_fusion(Sim &s, int L)
     }
     HIPCHK(hipStreamSynchronize(s.stream));
     l.fusedOpen = fuse;
-    return 0;
+    return prepare_images(s, l);
 }
 
 // rotor descriptors of a level to the device; the cell records follow at the next run
@@ -364,11 +404,35 @@ template <class S> static void settle_typed(Sim &s, Level &l)
     launch_open<S>(o, l.info.esotwistFlipper != 0, s.stream);
 }
 
+template <class S> static void periodic_typed(Sim &s, Level &l, bool flip)
+{
+    launch_periodic<S>(reinterpret_cast<S *>(l.f.p), topo_of(l), l.nPeriodic, l.perIndex.p, l.perSource.p, flip, s.stream);
+}
+
+// the periodic copy of ghosts that were stepped from their source cells
+static int settle_ghosts(Sim &s, Level &l)
+{
+    if (!l.ghostsStale) return 0;
+    l.ghostsStale = false;
+    const bool flip = l.info.esotwistFlipper != 0;
+    switch (s.storage) {
+    case LBM3_STORE_F16: periodic_typed<__half>(s, l, flip); break;
+    case LBM3_STORE_BF16: periodic_typed<__hip_bfloat16>(s, l, flip); break;
+    case LBM3_STORE_F16C: periodic_typed<f16c>(s, l, flip); break;
+    case LBM3_STORE_F64: periodic_typed<double>(s, l, flip); break;
+    default: periodic_typed<float>(s, l, flip); break;
+    }
+    return check_hip(hipGetLastError(), "periodic ghost copy");
+}
+
 // A condition is pending after a fused step and after a checkpoint load that
 // saved one; it is applied here whether or not the level currently fuses.
+// Ghosts that lag behind their sources are copied too: what follows reads the
+// level's whole state.
 static int settle_open(Sim &s, int L)
 {
     Level &l = s.L[L];
+    if (const int rc = settle_ghosts(s, l)) return rc;
     if (l.openSettled || l.nOpen == 0) {
         l.openSettled = true;
         return 0;
@@ -446,10 +510,17 @@ template <class S> static void step_level(Sim &s, int level)
     }
     const StepParam *slot = s.captureTable ? s.captureTable + s.captureSlot++ : nullptr;
     a.param = slot;
+    // The step after an initialisation, an upload or a read of the whole state
+    // takes the ghosts as they are: a caller may have written them.  A captured
+    // step keeps the copy, so that every replay is the same.
+    const bool images = l.imagesReady && !slot;
+    if (images && l.ghostsStale) {
+        a.fast.skip = l.ghostSkip.p;
+        a.fast.images = {l.imageSources.p, l.imageHead.p, l.imageInfo.p, l.imageNb.p};
+    }
     // side-stream choice 3: the wall-adjacent cells in blocks ahead of the bulk
-    // blocks of one launch (not with rotor cells in the bulk kernel, rotated
-    // lanes or 64-bit offsets)
-    const bool walls = s.tune.overlap == 3 && l.W > 0 && !a.fast.rotorBits && !a.laneRot && !wide_level<S>(l.N);
+    // blocks of one launch (not with rotated lanes or 64-bit offsets)
+    const bool walls = s.tune.overlap == 3 && l.W > 0 && !a.laneRot && !wide_level<S>(l.N);
     a.wallBlocks = walls ? (int)((l.W + 255) / 256) : 0;
     if (timed || !s.tune.overlap || ((l.W == 0 || walls) && a.open.count == 0 && a.rotorCellCount == 0)) {
         // in order on one stream, so that each kernel's events bracket it alone
@@ -498,7 +569,8 @@ template <class S> static void step_level(Sim &s, int level)
         o.param = slot;
         launch_open<S>(o, nflip, s.stream);
     }
-    launch_periodic<S>(reinterpret_cast<S *>(l.f.p), topo_of(l), l.nPeriodic, l.perIndex.p, l.perSource.p, nflip, s.stream);
+    if (images) l.ghostsStale = true;
+    else periodic_typed<S>(s, l, nflip);
     l.info.iterationsSinceTrackerReset++;
     l.info.iterationsFinished++;
 }
@@ -553,6 +625,7 @@ template <class S> static int init_level(Sim &s, int level, const float *fieldsD
     d.fields = fieldsDev;
     const bool flip = l.info.esotwistFlipper != 0;
     l.openSettled = true;
+    l.ghostsStale = false;
     launch_init<S>(reinterpret_cast<S *>(l.f.p), topo_of(l), d, l.geom, s.codec, flip, s.stream);
     launch_open_ref_init<S>(open_args<S>(s, l, l.info.iterationsFinished), l.info.cellCountX, l.info.cellCountY, l.info.cellCountZ, flip, s.stream);
     return check_hip(hipGetLastError(), "init kernels");
@@ -1000,6 +1073,7 @@ static int take_snapshot(Sim &s, Snapshot &z)
     z = Snapshot{};
     for (int L = 0; L < s.levels; ++L) {
         Level &l = s.L[L];
+        if (const int rc = settle_ghosts(s, l)) return rc;
         for (const auto &b : checkpoint_buffers(l, s.storage)) {
             z.bufs.emplace_back();
             if (b.second == 0 || !b.first) continue;
@@ -1032,6 +1106,7 @@ static int restore_snapshot(Sim &s, Snapshot &z)
         l.info.esotwistFlipper = z.infos[(size_t)L].esotwistFlipper;
         for (size_t r = 0; r < l.rotors.size(); ++r) l.rotors[r].radiansElapsed = z.angles[(size_t)L][r];
         l.openSettled = z.settled[(size_t)L] != 0;
+        l.ghostsStale = false;
     }
     return check_hip(hipStreamSynchronize(s.stream), "snapshot restore");
 }
@@ -1212,6 +1287,8 @@ int lbm3_run_graph(lbm3_sim *h, int steps)
     Sim &s = h->s;
     if (const int rc = check_run(s, 0)) return rc;
     if (s.timing) return set_error(LBM3_E_STATE, "graph replay during a timed run");
+    for (int L = 0; L < s.levels; ++L)
+        if (const int rc = settle_ghosts(s, s.L[L])) return rc;
     if (steps >= 2) {
         // Two coarse steps bring every level's esotwist parity back, so one
         // captured pair replays with the same kernel arguments.  What changes
@@ -1409,6 +1486,7 @@ int lbm3_upload_populations(lbm3_sim *h, int level, const void *in, long long by
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s.stream));
     s.L[level].openSettled = true;   // an uploaded state is complete
+    s.L[level].ghostsStale = false;
     return 0;
 }
 
@@ -1826,6 +1904,8 @@ int lbm3_save_checkpoint(lbm3_sim *h, const char *path)
     Sim &s = h->s;
     for (int L = 0; L < s.levels; ++L)
         if (const int rc = check_level(s, L)) return rc;
+    for (int L = 0; L < s.levels; ++L)
+        if (const int rc = settle_ghosts(s, s.L[L])) return rc;
     HIPCHK(hipStreamSynchronize(s.stream));
     FILE *fp = fopen(path, "wb");
     if (!fp) return set_error(LBM3_E_ARG, std::string("cannot open checkpoint file: ") + path);
@@ -1930,6 +2010,7 @@ int lbm3_load_checkpoint(lbm3_sim *h, const char *path)
         l.info.iterationsSinceTrackerReset = infos[(size_t)L].iterationsSinceTrackerReset;
         l.info.esotwistFlipper = infos[(size_t)L].esotwistFlipper;
         l.openSettled = settled[(size_t)L] != 0;
+        l.ghostsStale = false;
     }
     fclose(fp);
     s.fluidUpdates = updates;

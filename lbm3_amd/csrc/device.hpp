@@ -41,22 +41,59 @@ __device__ __forceinline__ void decode(const Topology &t, int cell, int (&nb)[8]
 // the row, first cell of the j+ row, of the k+ row, of the jk+ row}.  The
 // neighbour cells of a cell are then two dependent loads away instead of four.
 // The bulk kernel reads neither per-cell record: a bit per cell says whether
-// another kernel (or none) updates it, and the row of every 256th cell, with
-// the rows' first cells, gives the row of the others.
+// another kernel (or none) updates it, and the row of every 64th cell gives a
+// wave its first row (row_in_wave).
+struct PeriodicImages {
+    const uint64_t *sources;   // as FastTopo::skip: cells with ghosts; null: the ghosts are stepped as cells of their own
+    const int *head;           // [N] first ghost entry of a source cell
+    const int2 *info;          // per ghost entry {directions another cell reads, next entry of the same source or -1}
+    const int4 *nb;            // [2] per ghost entry: the ghost's eight neighbour cells
+};
+
 struct FastTopo {
     int N;
     const int2 *cellRow;   // [N]
-    const int4 *rows;      // [nRows]
+    const int4 *rows;      // [nRows + kRowPad], the last kRowPad starting past every cell
     const uint64_t *skip;  // [N / 64 rounded up to 4] bit c % 64 of word c / 64: not a bulk cell; null: read cellRow
-    const int *tileRow;    // [N / 256 rounded up] row of cell 256 t
+    const int *waveRow;    // [N / 64 rounded up to 4] row of cell 64 w
     int nRows;
     const uint64_t *openBits;  // as skip: open cells the bulk kernel completes and steps itself; null: none
     const uint64_t *rotorBits; // as skip: cells the rotors can reach, stepped by the bulk kernel; null: none
+    PeriodicImages images;     // the periodic ghosts are stepped by their source cells (skip then covers them)
 };
 
-__device__ __forceinline__ void decode_fast(const FastTopo &t, int cell, int row, int (&nb)[8])
+constexpr int kRowPad = 4;
+
+// The row of a lane's cell, its record in r, from the row r0 of the first cell
+// of its wave.  The wave's first four rows come in one scalar load (the table
+// is padded), and a wave that lies in one row, or in up to three, needs no
+// further load; only rows shorter than about 21 cells put more into a wave and
+// are searched lane by lane from there.  A loop of dependent loads over the
+// rows of a 256-cell block stood here before (up to eight in a row on a 32^3
+// box): 64^3 FP32 vortex 16.7 -> 14.8 us per step, 32^3 11.9 -> 10.6.
+__device__ __forceinline__ int row_in_wave(const FastTopo &t, int r0, int cell, int4 &r)
 {
-    const int4 r = t.rows[row];
+    const int4 *p = t.rows + r0;
+    const int4 a = p[0], b = p[1], c = p[2], d = p[3];
+    r = a;
+    const int last = __builtin_amdgcn_readfirstlane(cell | 63);
+    int row = r0;
+    if (last >= b.x) {
+        if (cell >= b.x) { r = b; row = r0 + 1; }
+        if (cell >= c.x) { r = c; row = r0 + 2; }
+        if (last >= d.x) {
+            if (cell >= d.x) {
+                row = r0 + 3;
+                while (t.rows[row + 1].x <= cell) ++row;
+                r = t.rows[row];
+            }
+        }
+    }
+    return row;
+}
+
+__device__ __forceinline__ void decode_row(const FastTopo &t, int cell, const int4 &r, int (&nb)[8])
+{
     const int back = cell - r.x;
     const int N = t.N;
     nb[0] = cell;
@@ -67,6 +104,12 @@ __device__ __forceinline__ void decode_fast(const FastTopo &t, int cell, int row
     nb[4] = nb[2] + 1 >= N ? 0 : nb[2] + 1;
     nb[5] = nb[3] + 1 >= N ? 0 : nb[3] + 1;
     nb[7] = nb[6] + 1 >= N ? 0 : nb[6] + 1;
+}
+
+__device__ __forceinline__ void decode_fast(const FastTopo &t, int cell, int row, int (&nb)[8])
+{
+    const int4 r = t.rows[row];
+    decode_row(t, cell, r, nb);
 }
 
 // getLocalBC resolved per (level, wallID): rules depend only on those two keys,
@@ -206,14 +249,14 @@ template <class S> struct OpenArgs {
 };
 
 // Blocks are dispatched round-robin over the 8 XCDs.  With bit 0 of the block
-// order each XCD gets a contiguous range of blocks (its own L2 then sees whole
-// neighbouring rows); with the tiled population layout the plain order, in
-// which the whole chip works on one narrow window of tiles at a time, measured
-// 4% faster on the 256x128x128 sphere bulk kernel (162 vs 169 us).  Bit 1
-// sweeps the tiles backwards on odd esotwist parity, so that each step starts
-// on the lines the previous step wrote last, still in the 256 MB last-level
-// cache: the FP32 sphere bulk kernel (452 MB of populations) 186 -> 158 us.
-// Default: plain order, reversed every other step.
+// order each XCD gets a contiguous range of blocks, whose rows and, from one
+// step to the next, whose populations its own L2 then holds.  Bit 1 sweeps the
+// tiles (of each XCD's range, or of the level) backwards on odd esotwist parity,
+// so that each step starts on the lines the previous step wrote last, still in
+// L2 and the 256 MB last-level cache: the FP32 sphere bulk kernel (452 MB of
+// populations) 186 -> 158 us.  Backwards within each range instead of over the
+// whole level keeps a range on its XCD: FP16 sphere 97.2 -> 93.6 us per step,
+// 64^3 vortex 16.7 -> 15.0.
 #ifndef LBM3_XCD_REMAP
 #define LBM3_XCD_REMAP 2
 #endif
@@ -230,17 +273,16 @@ template <class S> struct OpenArgs {
 
 // The tile a bulk block takes.  remap bit 0: blocks dealt so that each XCD
 // sweeps one contiguous part (else round-robin over the XCDs); bit 1: on odd
-// esotwist parity the tiles in reverse order, so that a step starts where the
-// previous one ended, on the lines the last-level cache still holds
+// esotwist parity each part (or the whole) in reverse order
 __device__ __forceinline__ int xcd_block(int b, int n, int remap, bool flip)
 {
-    int t = b;
+    const bool back = (remap & 2) && flip;
     if (remap & 1) {
-        const int per = n / 8;
-        if (b < per * 8) t = (b % 8) * per + b / 8;
+        // the leftover blocks past the eight parts keep their place at the end
+        const int per = n / 8, x = b / 8;
+        return b < per * 8 ? (b % 8) * per + (back ? per - 1 - x : x) : b;
     }
-    if ((remap & 2) && flip) t = n - 1 - t;
-    return t;
+    return back ? n - 1 - b : b;
 }
 
 } // namespace lbm3

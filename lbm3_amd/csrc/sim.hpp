@@ -67,13 +67,20 @@ struct Level {
     DBuf<int4> openNb;               // [2][nOpen] neighbour cells of each open cell
     DBuf<uint32_t> openMeta;
     DBuf<uint64_t> bulkSkip;         // per 64 cells: bit set where the bulk kernel leaves the cell to others
-    DBuf<int> tileRow;               // per 256 cells: row of the first cell
+    DBuf<int> waveRow;               // per 64 cells: row of the first cell
     DBuf<float> openScale;           // per open entry: velocity profile factor (null: no rule has a profile)
     DBuf<OpenBCRecord> openRecords;
     DBuf<unsigned char> openRefs;    // 2 arrays of nOpen compute-type values
     DBuf<double> openCum;            // 2 arrays of nOpen
     int nPeriodic = 0;
     DBuf<int> perIndex, perSource;
+    // the bulk kernel steps the periodic ghosts from their source cells (PeriodicImages)
+    bool imagesReady = false;        // the tables below are made, for the current cell records
+    bool ghostsStale = false;        // the ghosts' own populations lag behind their sources'
+    DBuf<uint64_t> ghostSkip, imageSources;
+    DBuf<int> imageHead;
+    DBuf<int2> imageInfo;
+    DBuf<int4> imageNb;
     InterfaceLists C2F, F2C;
     std::vector<int> fineRefs;       // imported lists: fine cells they name, checked against the finer level
     bool interfaceChecked = true;

@@ -360,32 +360,52 @@ __device__ __forceinline__ void open_in_bulk(const StepArgs<S> &a, int cell, typ
     }
 }
 
-template <class S, bool FLIP, int BULK, class Off, bool OPEN = false, bool ROTOR = false, bool ROT = false>
+// byte offset of a cell's slot run in its tile; the plane adds a wave-uniform
+// plane * TILE * sizeof(S)
+template <class S, class Off> __device__ __forceinline__ Off slot_offset(int cell)
+{
+    return (Off(uint32_t(cell) / LBM3_TILE) * Off(27 * LBM3_TILE) + Off(uint32_t(cell) % LBM3_TILE)) * Off(sizeof(S));
+}
+
+// IMG: a periodic ghost holds its source cell's populations, so it collides to
+// the same values and streams them into the cells beside it.  The source's
+// thread does that for it: after its own stores it writes its post-collision
+// populations to each ghost's slots too, those directions that a cell other
+// than a ghost reads.  The ghosts' own populations stay stale until something
+// reads them (settle_ghosts copies them then, as a pass after streaming does
+// where this is off).  Small boxes are bound by launches and the latency of one
+// wave: with the second launch gone a step of the 64^3 vortex takes 16.7 us
+// instead of 21.1 (FP32, fastest launch choices of each), FP16 106^3 37.0
+// instead of 43.2, the 256x64x64 duct in BF16 34.5 instead of 40.3; the rows of
+// a wave in one scalar load (row_in_wave) take them to 14.8, 35.1 and 32.7.
+template <class S, bool FLIP, int BULK, class Off, bool OPEN = false, bool ROTOR = false, bool ROT = false, bool IMG = false>
 __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell)
 {
     using T = typename StoreTraits<S>::compute;
+    // one mask word and one row per wave of 64 aligned cells, both scalar loads
     int row;
-    if (a.fast.skip) {
-        // a wave's 64 cells are 64-aligned and a block's 256: one mask word per
-        // wave and one row per block, both scalar loads
+    int4 r4;
+    if constexpr (ROT) {
+        // the lanes of a wave lie in two words
+        const int r0 = a.fast.waveRow[cell >> 6];
         if (mask_bit<ROT>(a.fast.skip, cell)) return;   // handled by another kernel, or solid
-        int r = a.fast.tileRow[__builtin_amdgcn_readfirstlane(cell >> 8)];
-        while (r + 1 < a.fast.nRows && a.fast.rows[r + 1].x <= cell) ++r;
-        row = r;
+        row = r0;
+        while (a.fast.rows[row + 1].x <= cell) ++row;
+        r4 = a.fast.rows[row];
     } else {
-        const long long rec = __builtin_nontemporal_load(reinterpret_cast<const long long *>(a.fast.cellRow) + cell);
-        const int wm = int(rec);
-        row = int(rec >> 32);
-        if (wm >= 0 || wm <= -3) return;   // handled by another kernel, or solid
+        const int r0 = a.fast.waveRow[__builtin_amdgcn_readfirstlane(cell >> 6)];
+        const uint64_t skip = a.fast.skip[__builtin_amdgcn_readfirstlane(cell >> 6)];
+        row = row_in_wave(a.fast, r0, cell, r4);
+        if ((skip >> (cell & 63)) & 1ull) return;
     }
+    int img = -1;
+    if constexpr (IMG)
+        if (mask_bit<ROT>(a.fast.images.sources, cell)) img = a.fast.images.head[cell];
     int nb[8];
-    decode_fast(a.fast, cell, row, nb);
-    // byte offset of each neighbour's slot run in its tile; the plane adds a
-    // wave-uniform plane * TILE * sizeof(S)
+    decode_row(a.fast, cell, r4, nb);
     Off off[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-        off[k] = (Off(uint32_t(nb[k]) / LBM3_TILE) * Off(27 * LBM3_TILE) + Off(uint32_t(nb[k]) % LBM3_TILE)) * Off(sizeof(S));
+    for (int k = 0; k < 8; ++k) off[k] = slot_offset<S, Off>(nb[k]);
     T f[27];
     if constexpr (sizeof(Off) == 4 && (sizeof(S) >= 4 || LBM3_BUF16 > 0)) {
         // raw buffer accesses: the plane offset is a scalar operand
@@ -393,12 +413,37 @@ __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell)
 #pragma unroll
         for (int q = 0; q < 27; ++q)
             f[q] = StoreTraits<S>::bload(r, off[pre_nb(q)], pre_plane(q, FLIP) * LBM3_TILE * int(sizeof(S)), q, a.cd);
+        int2 gi = {};
+        int4 g0 = {}, g1 = {};
+        if constexpr (IMG) {
+            if (img >= 0) {   // the first ghost's entry arrives during the collision
+                gi = a.fast.images.info[img];
+                g0 = a.fast.images.nb[2 * (size_t)img];
+                g1 = a.fast.images.nb[2 * (size_t)img + 1];
+            }
+        }
         open_in_bulk<S, OPEN, ROT>(a, cell, f);
         bulk_collide<S, BULK, ROTOR>(a, cell, row, f);
         if constexpr (sizeof(S) >= 4 || LBM3_BUF16 == 1) {
 #pragma unroll
             for (int q = 0; q < 27; ++q)
                 StoreTraits<S>::bstore(r, off[post_nb(q)], post_plane(q, FLIP) * LBM3_TILE * int(sizeof(S)), f[q], q, a.cd);
+            if constexpr (IMG) {
+                while (img >= 0) {
+                    const int gn[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+#pragma unroll
+                    for (int q = 1; q < 27; ++q)
+                        if ((gi.x >> q) & 1)
+                            StoreTraits<S>::bstore(r, slot_offset<S, Off>(gn[post_nb(q)]),
+                                                   post_plane(q, FLIP) * LBM3_TILE * int(sizeof(S)), f[q], q, a.cd);
+                    img = gi.y;
+                    if (img >= 0) {
+                        gi = a.fast.images.info[img];
+                        g0 = a.fast.images.nb[2 * (size_t)img];
+                        g1 = a.fast.images.nb[2 * (size_t)img + 1];
+                    }
+                }
+            }
         } else {
 #pragma unroll
             for (int q = 0; q < 27; ++q)
@@ -423,14 +468,14 @@ __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell)
 // row -- both x-face cells -- share one wave, which then runs the open
 // condition once for the two instead of two waves once each; every access of
 // that wave still fills whole 128-byte lines
-template <class S, bool FLIP, int BULK, bool WIDE, bool OPEN = false, bool ROTOR = false, bool ROT = false>
+template <class S, bool FLIP, int BULK, bool WIDE, bool OPEN = false, bool ROTOR = false, bool ROT = false, bool IMG = false>
 __global__ __launch_bounds__(256) void k_collide_stream(StepArgs<S> a)
 {
     const int lane = ROT ? int((threadIdx.x + 32) & 255) : int(threadIdx.x);
     const int cell = xcd_block(blockIdx.x, gridDim.x, a.xcdRemap, FLIP) * 256 + lane;
     if (cell >= a.fast.N) return;
     if (WIDE) bulk_cell<S, FLIP, BULK, uint64_t>(a, cell);
-    else bulk_cell<S, FLIP, BULK, uint32_t, OPEN, ROTOR, ROT>(a, cell);
+    else bulk_cell<S, FLIP, BULK, uint32_t, OPEN, ROTOR, ROT, IMG>(a, cell);
 }
 
 // Open-boundary cells (never wall-adjacent when this kernel is used): load,
@@ -486,10 +531,10 @@ static __global__ __launch_bounds__(256) void k_mark_groups(const int *groups, i
 }
 
 // the bulk kernel's view of the cell records: per 64 cells a mask of the cells
-// it skips (record >= 0 or <= -3, and the padding past N), per 256 cells the
-// row of the first one; with `open` non-null the open cells (record <= -8) are
+// it skips (record >= 0 or <= -3, and the padding past N) and the row of the
+// first one; with `open` non-null the open cells (record <= -8) are
 // the bulk kernel's too, marked in `open`
-static __global__ __launch_bounds__(256) void k_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *tileRow,
+static __global__ __launch_bounds__(256) void k_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *waveRow,
                                                    uint64_t *open, uint64_t *rotor)
 {
     const int cell = blockIdx.x * 256 + threadIdx.x;
@@ -507,15 +552,76 @@ static __global__ __launch_bounds__(256) void k_bulk_mask(const int2 *cellRow, i
         skip[cell >> 6] = m;
         if (open) open[cell >> 6] = o;
         if (rotor) rotor[cell >> 6] = q;
+        waveRow[cell >> 6] = row;
     }
-    if (threadIdx.x == 0) tileRow[blockIdx.x] = row;
 }
 
-LBM3_SHARED_DEF void launch_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *tileRow, uint64_t *open, uint64_t *rotor,
+LBM3_SHARED_DEF void launch_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *waveRow, uint64_t *open, uint64_t *rotor,
                       hipStream_t s)
 {
     if (N <= 0) return;
-    k_bulk_mask<<<(N + 255) / 256, 256, 0, s>>>(cellRow, N, skip, tileRow, open, rotor);
+    k_bulk_mask<<<(N + 255) / 256, 256, 0, s>>>(cellRow, N, skip, waveRow, open, rotor);
+}
+
+// Periodic ghosts stepped by their source cells (bulk_cell, IMG), on a level that is
+// one full box in x, y, z order.  Pass 0: every ghost and source must be a plain
+// bulk cell (record -1 or -2, where the box puts it), else *flag counts it;
+// the ghosts' skip bits and the sources' bits are set, the lists of the sources cleared.
+static __global__ __launch_bounds__(256) void k_image_marks(Topology t, FastTopo ft, int X, int Y, int count, const int *ghost,
+                                                            const int *source, uint64_t *skip, uint64_t *sources, int *head,
+                                                            int *flag)
+{
+    const int x = blockIdx.x * 256 + threadIdx.x;
+    if (x >= count) return;
+    const int c[2] = {ghost[x], source[x]};
+    for (int k = 0; k < 2; ++k) {
+        const int2 r = ft.cellRow[c[k]];
+        int ijk[3];
+        cell_ijk(t, ft, c[k], r.y, ijk);
+        if ((r.x != -1 && r.x != -2) || c[k] != ijk[0] + X * (ijk[1] + Y * ijk[2])) atomicAdd(flag, 1);
+    }
+    atomicOr(reinterpret_cast<unsigned long long *>(skip + (c[0] >> 6)), 1ull << (c[0] & 63));
+    atomicOr(reinterpret_cast<unsigned long long *>(sources + (c[1] >> 6)), 1ull << (c[1] & 63));
+    head[c[1]] = -1;
+}
+
+// pass 1: each ghost's neighbour cells, the directions whose post-collision
+// population a cell that is no ghost reads, and its place in its source's list
+// (any order: the ghosts' slots are disjoint)
+static __global__ __launch_bounds__(256) void k_image_lists(Topology t, FastTopo ft, int X, int Y, int Z, int count,
+                                                            const int *ghost, const int *source, const uint64_t *plainSkip,
+                                                            const uint64_t *skip, int *head, int2 *info, int4 *nbOut, int *flag)
+{
+    const int x = blockIdx.x * 256 + threadIdx.x;
+    if (x >= count) return;
+    const int g = ghost[x];
+    const int row = ft.cellRow[g].y;
+    int ijk[3], nb[8];
+    cell_ijk(t, ft, g, row, ijk);
+    decode_fast(ft, g, row, nb);
+    nbOut[2 * (size_t)x] = make_int4(nb[0], nb[1], nb[2], nb[3]);
+    nbOut[2 * (size_t)x + 1] = make_int4(nb[4], nb[5], nb[6], nb[7]);
+    auto is_ghost = [&](int c) { return ((skip[c >> 6] & ~plainSkip[c >> 6]) >> (c & 63)) & 1ull; };
+    if (is_ghost(source[x])) atomicAdd(flag, 1);   // a chain of ghosts
+    int dirs = 0;
+#pragma unroll
+    for (int q = 1; q < 27; ++q) {
+        const int i = ijk[0] + cx(q), j = ijk[1] + cy(q), k = ijk[2] + cz(q);
+        if (i < 0 || i >= X || j < 0 || j >= Y || k < 0 || k >= Z) continue;
+        if (!is_ghost(i + X * (j + Y * k))) dirs |= 1 << q;
+    }
+    info[x] = make_int2(dirs, atomicExch(&head[source[x]], x));
+}
+
+LBM3_SHARED_DEF void launch_images(const Topology &t, const FastTopo &ft, const LevelGeom &g, int count, const int *ghost,
+                                   const int *source, uint64_t *skip, uint64_t *sources, int *head, int2 *info, int4 *nb,
+                                   int *flag, hipStream_t s)
+{
+    if (count <= 0) return;
+    const unsigned b = (unsigned)((count + 255) / 256);
+    k_image_marks<<<b, 256, 0, s>>>(t, ft, g.cellCountX, g.cellCountY, count, ghost, source, skip, sources, head, flag);
+    k_image_lists<<<b, 256, 0, s>>>(t, ft, g.cellCountX, g.cellCountY, g.cellCountZ, count, ghost, source, ft.skip, skip, head,
+                                    info, nb, flag);
 }
 
 // the cells of the open groups leave the bulk kernel's view: skip bits set,
@@ -677,19 +783,16 @@ __device__ __noinline__ void wall_cell_call(const __attribute__((address_space(4
 // the bulk blocks, in one launch: no second stream and no join per step.  The
 // wall path needs about twice the bulk path's registers; the register budget is
 // held to six waves per SIMD (the bulk path fits it, the wall path spills), so
-// the bulk blocks keep their occupancy.  BF16 with the open cells inside: seven
-// waves (72 registers, no spill in the bulk path), measured on the
-// 256x128x128 sphere at 0.0988-0.0996 ms per step against 0.1012-0.1025 with
-// six; FP16 measured the other way round (0.0976-0.0990 with six, and seven
-// lost to the wall kernel on the side stream).
-template <class S>
-constexpr int walls_waves(bool open)
+// the bulk blocks keep their occupancy; at seven the 16-bit bulk path spills too.
+// With the rotor cells inside (103 registers) four waves: more would spill in
+// the rotor path.
+constexpr int walls_waves(bool rotor)
 {
-    return open && std::is_same<S, __hip_bfloat16>::value ? 7 : 6;
+    return rotor ? 4 : 6;
 }
 
-template <class S, bool FLIP, int BULK, bool OPEN>
-__global__ __launch_bounds__(256, walls_waves<S>(OPEN)) void k_collide_stream_walls(StepArgs<S> a)
+template <class S, bool FLIP, int BULK, bool OPEN, bool ROTOR = false>
+__global__ __launch_bounds__(256, walls_waves(ROTOR)) void k_collide_stream_walls(StepArgs<S> a)
 {
     const int b = blockIdx.x;
     if (b < a.wallBlocks) {
@@ -707,15 +810,15 @@ __global__ __launch_bounds__(256, walls_waves<S>(OPEN)) void k_collide_stream_wa
     }
     const int cell = xcd_block(b - a.wallBlocks, gridDim.x - a.wallBlocks, a.xcdRemap, FLIP) * 256 + threadIdx.x;
     if (cell >= a.fast.N) return;
-    bulk_cell<S, FLIP, BULK, uint32_t, OPEN>(a, cell);
+    bulk_cell<S, FLIP, BULK, uint32_t, OPEN, ROTOR>(a, cell);
 }
 
 // derive the hot-loop topology records from the compressed IJK/NBR arrays;
 // with rotorCand, the fluid cells the rotors can reach get -4, and with openOf
 // the open-boundary cells get -(8 + open-list index), in place of
 // their wall-map code (they are never wall-adjacent when this is used)
-static __global__ __launch_bounds__(256) void k_fast_topo(Topology t, const int *wallMap, const int *openOf, const uint8_t *rotorCand,
-                                                   int2 *cellRow, int4 *rows)
+static __global__ __launch_bounds__(256) void k_fast_topo(Topology t, int nRows, const int *wallMap, const int *openOf,
+                                                          const uint8_t *rotorCand, int2 *cellRow, int4 *rows)
 {
     const int cell = blockIdx.x * 256 + threadIdx.x;
     if (cell >= t.N) return;
@@ -725,6 +828,8 @@ static __global__ __launch_bounds__(256) void k_fast_topo(Topology t, const int 
     if (rotorCand && rotorCand[cell] && code >= -2 && code < 0) code = -4;
     if (openOf && openOf[cell] >= 0) code = -(8 + openOf[cell]);
     cellRow[cell] = make_int2(code, row);
+    if (cell == 0)
+        for (int k = 0; k < kRowPad; ++k) rows[nRows + k] = make_int4(0x7FFFFFFF, 0, 0, 0);   // past every cell (row_in_wave)
     if (shift >= 0) rows[row] = make_int4(cell, t.rjp[row], t.rkp[row], t.rjkp[row]);
 }
 
@@ -1190,11 +1295,17 @@ void launch_collide_stream(const StepArgs<S> &a, bool flip, hipStream_t s)
     const bool k17 = relax_of<typename StoreTraits<S>::compute>(a.bulk).k17 != 0;
     const bool wide = wide_level<S>(a.fast.N);
     if (a.wallBlocks > 0) {
-        // the caller combines only levels without rotor cells in the bulk
-        // kernel, rotated lanes or 64-bit offsets
+        // the caller combines only levels without rotated lanes or 64-bit offsets
         const dim3 gw(blocks_for(a.fast.N) + (unsigned)a.wallBlocks);
 #define LBM3_BULK_WALLS(F, K, O) hipLaunchKernelGGL((k_collide_stream_walls<S, F, K, O>), gw, b, lds, s, a)
+#define LBM3_BULK_WALLS_ROTOR(F, K) hipLaunchKernelGGL((k_collide_stream_walls<S, F, K, false, true>), gw, b, lds, s, a)
         const bool o = a.fast.openBits != nullptr;
+        if (a.fast.rotorBits) {
+            if (flip) { if (k17) LBM3_BULK_WALLS_ROTOR(true, 1); else LBM3_BULK_WALLS_ROTOR(true, 2); }
+            else { if (k17) LBM3_BULK_WALLS_ROTOR(false, 1); else LBM3_BULK_WALLS_ROTOR(false, 2); }
+            return;
+        }
+#undef LBM3_BULK_WALLS_ROTOR
         if (flip) { if (k17) { if (o) LBM3_BULK_WALLS(true, 1, true); else LBM3_BULK_WALLS(true, 1, false); }
                     else { if (o) LBM3_BULK_WALLS(true, 2, true); else LBM3_BULK_WALLS(true, 2, false); } }
         else { if (k17) { if (o) LBM3_BULK_WALLS(false, 1, true); else LBM3_BULK_WALLS(false, 1, false); }
@@ -1205,8 +1316,16 @@ void launch_collide_stream(const StepArgs<S> &a, bool flip, hipStream_t s)
 #define LBM3_BULK_LAUNCH(F, K, W) hipLaunchKernelGGL((k_collide_stream<S, F, K, W>), g, b, lds, s, a)
 #define LBM3_BULK_OPEN(F, K) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, true>), g, b, lds, s, a)
 #define LBM3_BULK_OPEN_ROT(F, K) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, true, false, true>), g, b, lds, s, a)
+#define LBM3_BULK_IMG(F, K, O) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, O, false, false, true>), g, b, lds, s, a)
 #define LBM3_BULK_ROTOR(F, K) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, false, true>), g, b, lds, s, a)
-    if (a.fast.rotorBits && !wide) {
+    if (a.fast.images.sources) {
+        // the level is neither wide nor has rotor cells, rotated lanes or wall-adjacent cells (prepare_images)
+        const bool o = a.fast.openBits != nullptr;
+        if (flip) { if (k17) { if (o) LBM3_BULK_IMG(true, 1, true); else LBM3_BULK_IMG(true, 1, false); }
+                    else { if (o) LBM3_BULK_IMG(true, 2, true); else LBM3_BULK_IMG(true, 2, false); } }
+        else { if (k17) { if (o) LBM3_BULK_IMG(false, 1, true); else LBM3_BULK_IMG(false, 1, false); }
+               else { if (o) LBM3_BULK_IMG(false, 2, true); else LBM3_BULK_IMG(false, 2, false); } }
+    } else if (a.fast.rotorBits && !wide) {
         if (flip) { if (k17) LBM3_BULK_ROTOR(true, 1); else LBM3_BULK_ROTOR(true, 2); }
         else { if (k17) LBM3_BULK_ROTOR(false, 1); else LBM3_BULK_ROTOR(false, 2); }
     } else if (a.fast.openBits && !wide && a.laneRot) {
@@ -1226,6 +1345,7 @@ void launch_collide_stream(const StepArgs<S> &a, bool flip, hipStream_t s)
 #undef LBM3_BULK_OPEN
 #undef LBM3_BULK_OPEN_ROT
 #undef LBM3_BULK_ROTOR
+#undef LBM3_BULK_IMG
 }
 
 template <class S>
@@ -1281,11 +1401,12 @@ LBM3_SHARED_DEF void launch_open_nb(const Topology &t, int count, const int *cel
     hipLaunchKernelGGL(k_open_nb, dim3(blocks_for(count)), dim3(256), 0, s, t, count, cell, out);
 }
 
-LBM3_SHARED_DEF void launch_fast_topo(const Topology &t, const int *wallMap, const int *openOf, const uint8_t *rotorCand, int2 *cellRow,
-                      int4 *rows, hipStream_t s)
+LBM3_SHARED_DEF void launch_fast_topo(const Topology &t, int nRows, const int *wallMap, const int *openOf, const uint8_t *rotorCand,
+                                      int2 *cellRow, int4 *rows, hipStream_t s)
 {
     if (t.N <= 0) return;
-    hipLaunchKernelGGL(k_fast_topo, dim3(blocks_for(t.N)), dim3(256), 0, s, t, wallMap, openOf, rotorCand, cellRow, rows);
+    hipLaunchKernelGGL(k_fast_topo, dim3(blocks_for(t.N)), dim3(256), 0, s, t, nRows, wallMap, openOf, rotorCand,
+                       cellRow, rows);
 }
 
 LBM3_SHARED_DEF void launch_open_conflicts(const int *cells, int count, int mode, const int *openOf, const int *wallMap,

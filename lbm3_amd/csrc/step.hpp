@@ -87,12 +87,16 @@ int launch_open_stats(const double *dRhoCum, const double *uNormalCum, const uin
                       double invSpan, double *partial, hipStream_t s);
 void launch_open_scale(const Topology &t, const LevelGeom &g, int count, const int *cell, const uint32_t *meta,
                        const OpenProfiles &P, float *scale, hipStream_t s);
-void launch_fast_topo(const Topology &t, const int *wallMap, const int *openOf, const uint8_t *rotorCand, int2 *cellRow,
+void launch_fast_topo(const Topology &t, int nRows, const int *wallMap, const int *openOf, const uint8_t *rotorCand, int2 *cellRow,
                       int4 *rows, hipStream_t s);
 void launch_scatter_index(const int *cell, int count, int *openOf, hipStream_t s);
 void launch_scatter_entries(const int *cell, const int *list, int count, int *openOf, hipStream_t s);
-void launch_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *tileRow, uint64_t *open, uint64_t *rotor,
+void launch_bulk_mask(const int2 *cellRow, int N, uint64_t *skip, int *waveRow, uint64_t *open, uint64_t *rotor,
                       hipStream_t s);
+// the lists by which the bulk kernel steps the periodic ghosts of a full box from their source
+// cells: `skip` comes in as a copy of ft.skip, `sources` zeroed; *flag counts what forbids it
+void launch_images(const Topology &t, const FastTopo &ft, const LevelGeom &g, int count, const int *ghost, const int *source,
+                   uint64_t *skip, uint64_t *sources, int *head, int2 *info, int4 *nb, int *flag, hipStream_t s);
 void launch_group_bits(const int *groups, int count, int G, uint64_t *skip, uint64_t *open, hipStream_t s);
 void launch_mark_groups(const int *groups, int count, int G, int N, int2 *cellRow, hipStream_t s);
 void launch_rotor_reach(const Topology &t, const LevelGeom &g, const RotorReachSet &R, uint8_t *cand, hipStream_t s);

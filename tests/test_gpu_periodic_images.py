@@ -1,0 +1,92 @@
+"""Periodic ghosts stepped by their source cells (one launch per step) against
+the copy after every step, on the GPU: the same populations bit for bit.  A
+captured step (run_graph) keeps the copy, so a replayed run is the copy path."""
+import numpy as np
+import pytest
+
+from lbm3_amd import cases, lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _make(case, dom, tris, storage, seed):
+    s = lib.Sim(case, storage)
+    s.build(dom, tris)
+    n = s.info(0).cellCount
+    r = np.random.RandomState(seed)
+    # ghosts hold values of their own at the start, unlike their sources'
+    f = (r.rand(n, 4).astype(np.float32) - 0.5) * np.array([0.002, 0.04, 0.04, 0.04], np.float32)
+    s.init_fields(0, f)
+    return s
+
+
+BOXES = {
+    "cube 4": lambda: cases.periodic_box(4),           # every cell a source of several ghosts
+    "cube 14": lambda: cases.periodic_box(14),
+    "cube 30 K17": lambda: cases.periodic_box(30, nu=0.02, limiter=0.1),
+    "cube 62": lambda: cases.periodic_box(62),         # rows of a whole wave
+    "duct": lambda: cases.channel(20, 12, 10),         # open cells beside the ghosts
+    "plane channel": lambda: cases.channel(26, 8, 18, periodic_z=True),
+}
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64", "f16", "bf16", "f16c"])
+@pytest.mark.parametrize("box", list(BOXES))
+def test_images_equal_the_copy(box, storage):
+    a, b = (_make(*BOXES[box](), storage, 3) for _ in range(2))
+    for steps in (1, 2, 5, 4):
+        a.run(steps)
+        b.run_graph(steps)
+        got, last = a.populations(0), b.populations(0)
+        assert got.tobytes() == last.tobytes(), (steps, np.argwhere(got.view(np.uint8) != last.view(np.uint8))[:4])
+    a.run(3)
+    b.run(3)
+    assert a.macros(0).tobytes() == b.macros(0).tobytes()
+    assert a.kinetic_energy() == b.kinetic_energy()
+
+
+def test_images_with_open_cells_in_the_bulk_kernel():
+    """Open cells completed by the bulk kernel (group width 1) beside ghosts."""
+    sims = []
+    for group in (1, 8):
+        s = _make(*BOXES["duct"](), "f32", 5)
+        s.run(1)
+        s.set_tune(0, 2, 1, group)
+        s.run(12)
+        sims.append(s)
+    assert sims[0].populations(0).tobytes() == sims[1].populations(0).tobytes()
+
+
+def test_images_checkpoint_and_graph(tmp_path):
+    """Stale ghosts are copied before a checkpoint is written and before a capture."""
+    a, b = (_make(*BOXES["cube 14"](), "f32", 9) for _ in range(2))
+    a.run(5)
+    b.run(5)
+    a.save_checkpoint(tmp_path / "c")
+    a.run(4)
+    a.run_graph(7)
+    a.run(3)
+    b.run(14)
+    assert a.populations(0).tobytes() == b.populations(0).tobytes()
+    a.load_checkpoint(tmp_path / "c")
+    a.run(14)
+    assert a.populations(0).tobytes() == b.populations(0).tobytes()
+
+
+@pytest.mark.parametrize("n", [4, 6, 18, 30])
+def test_short_rows_equal_the_oracle(n):
+    """Rows of 6 to 32 cells (several to a wave, the table's padding within
+    reach of the last wave) in FP64 against the oracle, ghosts included."""
+    from tests.helpers import rel_max
+    from tests.oracle_lib import OracleSim
+    case, dom, tris = cases.periodic_box(n, u=(0.02, 0.01, -0.005))
+    o = OracleSim(case, dom, tris, double=True)
+    s = lib.Sim(case, "f64")
+    s.build(dom, tris)
+    f = (np.random.RandomState(n).rand(s.info(0).cellCount, 4) - 0.5) * np.array([0.002, 0.04, 0.04, 0.04])
+    o.init_fields(0, f.astype(np.float32))
+    s.init_fields(0, f.astype(np.float32))
+    o.run(21)
+    s.run(21)
+    a, b = o.macros(), s.macros(0)
+    assert max(rel_max(1 + b[:, 0], 1 + a[:, 0]), rel_max(b[:, 1:], a[:, 1:])) < 1e-10
