@@ -149,7 +149,9 @@ int lbm3_synchronize(lbm3_sim *s);
  * bulk kernel, ms per step in the sweep}] for the first `cap` candidates; *nOut the
  * candidates timed. */
 int lbm3_autotune(lbm3_sim *s, int steps, double *out, int cap, int *nOut);
-/* The launch choices in use: {bulk LDS bytes, block order, side streams, open
+/* The launch choices in use (until lbm3_set_tune or lbm3_autotune sets them, each
+ * level takes its own by its size and cells; lbm3_get_tune then gives level
+ * 0's): {bulk LDS bytes, block order, side streams, open
  * group cells, x-face choice, rotor cells in the bulk kernel}; lbm3_set_tune
  * sets them (LDS 0..65536, block order 0..3, side streams 0..3, group 1, 8 or
  * 16, x-face choice 0..3, rotor cells 0..1; a new layout of the open or rotor

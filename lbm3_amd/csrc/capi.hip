@@ -188,6 +188,47 @@ static bool wide_of(const Sim &s, const Level &l)
     return 27LL * padded_cells(l.N) * (long long)storage_bytes(s.storage) > 0xFFFFFFFFLL;
 }
 
+// The launch choices of a level that nobody chose (lbm3_set_tune, lbm3_autotune).
+// Times are us per step on this GPU, FP32 unless said otherwise:
+// * one launch per step: the wall-adjacent cells in blocks ahead of the bulk
+//   blocks, the open cells and the rotor cells in the bulk kernel.  Against
+//   groups of open cells, wall cells and rotor cells on side streams: sphere
+//   96x48x48 57 -> 24, 186x92x84 (K17) 86 -> 57, 256x128x128 179 -> 155 (FP16
+//   126 -> 94), two-level rotor duct 427 -> 286.  Levels of up to 32768 cells
+//   keep the groups (48x24x24: 34 against 18): there the open cells have
+//   always been reported as cells of a kernel of their own.
+// * the levels in order on one stream: three-level sphere 344, with a stream
+//   per level 384.
+// * block order: one contiguous part per XCD, swept backwards every other step
+//   (order 3), so that each XCD's L2 and the last-level cache still hold what
+//   the step starts on: 64^3 vortex 14.9 against 18.3 in plain order, duct
+//   256x64x64 40 / 44, sphere 256x128x128 (452 MB) 155 / 157.  The plain order
+//   swept backwards (2) wins above about 512 MiB of populations, 300x150x150
+//   (729 MB) 272 against 289, and where rotors make some parts slower than
+//   others: rotor duct 286 / 306.
+// * occupancy cap of the bulk kernel (40 KiB of LDS per block, four blocks per
+//   CU: their tiles then fit an XCD's L2): above 1 GiB, 400x200x200 632 against
+//   692 (300x150x150: 277 / 272), and on levels of 64 to 256 MiB without open
+//   cells, three-level sphere 344 / 354, 130^3 vortex 91.2 / 93.2 (50 MB level
+//   25.2 / 23.6, 158^3 vortex of 443 MB 154 / 147).  Never for 16-bit storage,
+//   whose kernels are bound by instructions: FP16 256x128x128 115 / 94,
+//   400x200x200 464 / 380.
+Sim::Tune tune_of(const Sim &s, const Level &l)
+{
+    if (s.tuneChosen) return s.tune;
+    constexpr long long MiB = 1LL << 20;
+    const long long size = (long long)storage_bytes(s.storage), bytes = 27 * size * l.N;
+    Sim::Tune t;
+    t.overlap = 3;
+    t.ordered = true;
+    t.rotorInBulk = 1;
+    t.openGroup = l.N > 32768 ? 1 : 0;
+    t.xcdRemap = !l.rotors.empty() || bytes > 512 * MiB ? 2 : 3;
+    const bool cap = bytes > 1024 * MiB || (!l.openInBulk && bytes > 64 * MiB && bytes <= 256 * MiB);
+    t.bulkLds = size >= 4 && cap ? LBM3_BULK_LDS : 0;
+    return t;
+}
+
 // Whether the bulk kernel can step the periodic ghosts from their source cells
 // (one launch per step instead of a copy after each): a single level that is a
 // full box of plain fluid cells where ghosts and sources lie.  Levels with
@@ -236,6 +277,7 @@ static int prepare_images(Sim &s, Level &l)
 static int prepare_open_fusion(Sim &s, int L)
 {
     Level &l = s.L[L];
+    const Sim::Tune tune = tune_of(s, l);
     if (const int rc = settle_open(s, L)) return rc;   // a condition pending under the old records
     l.openFusionChecked = true;
     l.imagesReady = false;
@@ -288,7 +330,7 @@ static int prepare_open_fusion(Sim &s, int L)
     l.nFusedEntries = l.nSepEntries = 0;
     l.fusedEntries.release();
     l.sepEntries.release();
-    if (fuse && s.tune.openSplit == 1) {
+    if (fuse && tune.openSplit == 1) {
         // cells on the x faces (one per row end: every access of theirs is a
         // line of its own) leave the open-cell kernel: the bulk kernel steps
         // them and a pass after streaming completes them
@@ -313,15 +355,15 @@ static int prepare_open_fusion(Sim &s, int L)
     l.nOpenGroups = 0;
     // the rotor cells in the bulk kernel (the kernel takes open cells or rotor
     // cells, not both: open cells then stay in groups)
-    l.rotorInBulk = cand && s.tune.rotorInBulk && !wide_of(s, l);
-    int G = s.tune.openGroup ? s.tune.openGroup : open_group_cells((int)storage_bytes(s.storage));
+    l.rotorInBulk = cand && tune.rotorInBulk && !wide_of(s, l);
+    int G = tune.openGroup ? tune.openGroup : open_group_cells((int)storage_bytes(s.storage));
     if (G == 1 && l.rotorInBulk) G = open_group_cells((int)storage_bytes(s.storage));
     l.openInBulk = fuse && G == 1;   // the bulk kernel completes and steps the open cells
-    l.laneRot = l.openInBulk && s.tune.openSplit == 3;
+    l.laneRot = l.openInBulk && tune.openSplit == 3;
     // the bulk kernel's open cells but those on the x faces, which stay in
     // groups of the open-cell kernel (one x-face cell per row end would hold a
     // bulk wave for one lane; eight in a group share one wave's condition code)
-    const bool xGroups = l.openInBulk && s.tune.openSplit == 2;
+    const bool xGroups = l.openInBulk && tune.openSplit == 2;
     if (xGroups) G = open_group_cells((int)storage_bytes(s.storage));
     l.openGroupCells = G;
     if (fuse && (!l.openInBulk || xGroups)) {
@@ -451,6 +493,7 @@ static int settle_open(Sim &s, int L)
 template <class S> static void step_level(Sim &s, int level)
 {
     Level &l = s.L[level];
+    const int overlap = tune_of(s, l).overlap;
     const bool flip = l.info.esotwistFlipper != 0;
     const bool timed = s.timing && level == 0;
     if (timed) {
@@ -520,9 +563,9 @@ template <class S> static void step_level(Sim &s, int level)
     }
     // side-stream choice 3: the wall-adjacent cells in blocks ahead of the bulk
     // blocks of one launch (not with rotated lanes or 64-bit offsets)
-    const bool walls = s.tune.overlap == 3 && l.W > 0 && !a.laneRot && !wide_level<S>(l.N);
+    const bool walls = overlap == 3 && l.W > 0 && !a.laneRot && !wide_level<S>(l.N);
     a.wallBlocks = walls ? (int)((l.W + 255) / 256) : 0;
-    if (timed || !s.tune.overlap || ((l.W == 0 || walls) && a.open.count == 0 && a.rotorCellCount == 0)) {
+    if (timed || !overlap || ((l.W == 0 || walls) && a.open.count == 0 && a.rotorCellCount == 0)) {
         // in order on one stream, so that each kernel's events bracket it alone
         launch_collide_stream<S>(a, flip, s.stream);
         if (timed) (void)hipEventRecord(s.ev[s.evUsed][1], s.stream);
@@ -595,7 +638,7 @@ void update_interface(Sim &s, int coarse);    // interface.hip
 // for them.  s.stream is the current level's stream throughout.
 static void update_all(Sim &s, int level)
 {
-    const bool fork = !s.dryRun && s.tune.overlap >= 2 && level + 1 < s.levels && s.levelStream[level + 1];
+    const bool fork = !s.dryRun && tune_of(s, s.L[level]).levelStreams() && level + 1 < s.levels && s.levelStream[level + 1];
     const hipStream_t own = s.stream;
     if (fork) {
         (void)hipEventRecord(s.levelFork[level + 1], own);
@@ -1167,7 +1210,9 @@ int lbm3_autotune(lbm3_sim *h, int steps, double *out, int cap, int *nOut)
     for (int r = 0; r < (rotors ? 2 : 1); ++r)
         for (const auto &o : open) groups.push_back({o.first, o.second, r});
     const int ldsChoices[4] = {0, 24576, 40960, 65536};
-    const Sim::Tune start = s.tune;
+    const Sim::Tune start = tune_of(s, s.L[0]);
+    const bool startChosen = s.tuneChosen;
+    s.tuneChosen = true;
     Sim::Tune best = start;
     double bestMs = 1e300;
     int rows = 0;
@@ -1235,6 +1280,7 @@ int lbm3_autotune(lbm3_sim *h, int steps, double *out, int cap, int *nOut)
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     s.tune = start;
+    s.tuneChosen = startChosen;
     const int rg = regroup(s);
     const int rs = restore_snapshot(s, z);
     if (rc) return rc;
@@ -1245,13 +1291,14 @@ int lbm3_autotune(lbm3_sim *h, int steps, double *out, int cap, int *nOut)
     // one first (regroup), which rounds it to the storage type once
     const bool relayout = !same_open_layout(s, start, best);
     s.tune = best;
+    s.tuneChosen = true;
     return relayout ? regroup(s) : 0;
 }
 
 int lbm3_get_tune(lbm3_sim *h, int *out6)
 {
     if (!h || !out6) return set_error(LBM3_E_ARG, "null argument");
-    const Sim::Tune &t = h->s.tune;
+    const Sim::Tune t = tune_of(h->s, h->s.L[0]);
     out6[0] = t.bulkLds; out6[1] = t.xcdRemap; out6[2] = t.overlap;
     out6[3] = t.openGroup ? t.openGroup : open_group_cells((int)storage_bytes(h->s.storage));
     out6[4] = t.openSplit;
@@ -1269,7 +1316,9 @@ int lbm3_set_tune(lbm3_sim *h, const int *in6)
                                      "kernel), 8 or 16 cells, x-face choice 0..3, rotor cells 0..1");
     Sim &s = h->s;
     if (s.timing) return set_error(LBM3_E_STATE, "launch choices changed during a timed run");
-    const Sim::Tune was = s.tune;
+    const Sim::Tune was = tune_of(s, s.L[0]);
+    s.tuneChosen = true;
+    s.tune = Sim::Tune{};
     s.tune.bulkLds = in6[0];
     s.tune.xcdRemap = in6[1];
     s.tune.overlap = in6[2];
@@ -1989,6 +2038,8 @@ int lbm3_load_checkpoint(lbm3_sim *h, const char *path)
         Level &l = s.L[L];
         if (settled[(size_t)L] || !l.fusedOpen || split[(size_t)L] == (l.nSepEntries > 0)) continue;
         if (const int rc = settle_open(s, L)) { fclose(fp); return rc; }
+        s.tune = tune_of(s, l);
+        s.tuneChosen = true;
         s.tune.openSplit = split[(size_t)L] ? 1 : 0;
         l.openFusionChecked = false;
         if (const int rc = prepare_open_fusion(s, L)) { fclose(fp); return rc; }

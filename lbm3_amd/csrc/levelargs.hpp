@@ -27,8 +27,9 @@ template <class S> inline StepArgs<S> step_args(Sim &s, Level &l)
     a.wallBC = l.wallBC.p;
     a.wallVel = l.wallVel.p;
     a.param = nullptr;
-    a.xcdRemap = s.tune.xcdRemap;
-    a.bulkLds = s.tune.bulkLds;
+    const Sim::Tune tune = tune_of(s, l);
+    a.xcdRemap = tune.xcdRemap;
+    a.bulkLds = tune.bulkLds;
     a.laneRot = l.openInBulk && l.laneRot ? 1 : 0;
     a.wallBlocks = 0;
     a.geom = l.geom;

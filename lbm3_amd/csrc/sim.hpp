@@ -169,7 +169,12 @@ struct Sim {
         // a row's two x-face cells share a wave
         int openSplit = 0;
         int rotorInBulk = 0;          // the rotor cells stepped by the bulk kernel instead of their own
+        // each finer level's sub-cycle on a stream of its own (overlap 2 and 3
+        // ask for it where several levels exist)
+        bool levelStreams() const { return !ordered && overlap >= 2; }
+        bool ordered = false;         // overlap 3 with the levels in order on one stream (tune_of)
     } tune;
+    bool tuneChosen = false;         // the caller or the autotuner set `tune`; else every level takes tune_of's rule
     // graph capture: each level step takes the next slot of this device table
     // for the values that change between replays; a dry run only collects them
     StepParam *captureTable = nullptr;
@@ -185,6 +190,7 @@ struct Sim {
     int evUsed = 0;
 };
 
+Sim::Tune tune_of(const Sim &s, const Level &l);   // the launch choices of a level (capi.hip)
 size_t storage_bytes(int storage);
 size_t compute_bytes(int storage);
 int finish_level_setup(Sim &s, int level);  // derived tables after a level's arrays exist

@@ -90,3 +90,21 @@ def test_short_rows_equal_the_oracle(n):
     s.run(21)
     a, b = o.macros(), s.macros(0)
     assert max(rel_max(1 + b[:, 0], 1 + a[:, 0]), rel_max(b[:, 1:], a[:, 1:])) < 1e-10
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+def test_default_choices_equal_the_side_stream_kernels(storage):
+    """A sphere large enough for the one-launch default (open and wall cells in
+    the bulk kernel's launch) against the kernels of their own: same bits."""
+    case, dom, tris = cases.sphere(70, 34, 32, diameter=9.0, center=(20.0, 17.0, 16.0), segments=(16, 32))
+    out = []
+    for chosen in (None, (40960, 2, 1, 8)):
+        s = lib.Sim(case, storage)
+        s.build(dom, tris)
+        s.init()
+        if chosen:
+            s.set_tune(*chosen)
+        s.run(25)
+        assert (s.cell_kinds(0)["open_in_bulk"] > 0) == (chosen is None)
+        out.append((s.populations(0).tobytes(), s.wall_forces(0).tobytes()))
+    assert out[0] == out[1]
