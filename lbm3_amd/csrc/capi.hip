@@ -56,6 +56,7 @@ Codec make_codec(const lbm3_case &c, int storage)
             k.iw[q] = std::ldexp(k.iw[q], -112);
         }
     }
+    for (int a = 0; a < 3; ++a) k.u[a] = c.storeRef[a];
     return k;
 }
 

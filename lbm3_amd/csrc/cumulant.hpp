@@ -147,6 +147,104 @@ __host__ __device__ __forceinline__ void from_central_moments(T (&f)[27], const 
     cm_backward(a_cc0, a_cc1, a_cc2, uz, uz2, W36, f[PPM], f[PPO], f[PPP]);
 }
 
+// central moments up to third order (well-conditioned: the weights' own are taken off)
+template <class T> struct LowMoments {
+    T k100, k010, k001, k200, k020, k002, k110, k101, k011;
+    T k120, k102, k210, k012, k201, k021, k111;
+};
+
+// the relaxation: pre-collision moments up to third order -> all post-collision
+// central moments.  MODE as in collide.
+template <class T, int MODE>
+__host__ __device__ __forceinline__ CentralMoments<T> relax_moments(const LowMoments<T> &K, T dRho, T rho, T rhoInv, T ux2, T uy2,
+                                                                    T uz2, const Relax<T> &R)
+{
+    constexpr T third = T(1) / T(3), ninth = T(1) / T(9);
+    const T k100 = K.k100, k010 = K.k010, k001 = K.k001, k200 = K.k200, k020 = K.k020, k002 = K.k002;
+    const T k110 = K.k110, k101 = K.k101, k011 = K.k011;
+    const T k120 = K.k120, k102 = K.k102, k210 = K.k210, k012 = K.k012, k201 = K.k201, k021 = K.k021, k111 = K.k111;
+    // fourth-order cumulants relax to their equilibrium (rate 1): their
+    // pre-collision values, and the fourth-order moments, are not needed
+    const T dRhoNinth = dRho * rhoInv * ninth;
+
+    // ---- relaxation ----
+    const T w1 = R.w1;
+    const T hr = T(0.5) * rhoInv;
+    const T Dxu = -w1 * hr * (T(2) * k200 - k020 - k002) - hr * (k200 + k020 + k002 - dRho);
+    const T Dyv = Dxu + T(1.5) * w1 * rhoInv * (k200 - k020);
+    const T Dzw = Dxu + T(1.5) * w1 * rhoInv * (k200 - k002);
+    const T DxvDyu = -T(3) * w1 * rhoInv * k110;
+    const T DxwDzu = -T(3) * w1 * rhoInv * k101;
+    const T DywDzv = -T(3) * w1 * rhoInv * k011;
+
+    const T om1 = T(1) - w1;
+    const T s110 = om1 * k110, s101 = om1 * k101, s011 = om1 * k011;
+    const T g1 = T(3) * rho * (T(1) - T(0.5) * w1);
+    const T g2 = T(1.5) * rho;   // 3 rho (1 - omega2/2), omega2 = 1
+    const T e33 = om1 * (k200 - k020) - g1 * (ux2 * Dxu - uy2 * Dyv);
+    const T e34 = om1 * (k200 - k002) - g1 * (ux2 * Dxu - uz2 * Dzw);
+    const T e35 = dRho - g2 * (ux2 * Dxu + uy2 * Dyv + uz2 * Dzw);
+    const T s200 = (e33 + e34 + e35) * third;
+    const T s020 = (e34 - T(2) * e33 + e35) * third;
+    const T s002 = (e33 - T(2) * e34 + e35) * third;
+
+    T s120 = 0, s102 = 0, s210 = 0, s012 = 0, s201 = 0, s021 = 0, s111 = 0;
+    T c220 = 0, c202 = 0, c022 = 0, c211 = 0, c121 = 0, c112 = 0;
+    const bool k17 = MODE == 1 || (MODE == 0 && R.k17);
+    if (MODE != 2 && k17) {
+        const T lambda = R.lambda;
+        // limited relaxation: the rate tends to 1 where the cumulant is large compared to lambda
+        auto limited = [&](T c, T w) {
+            const T a = c < T(0) ? -c : c;
+            const T wl = w + (T(1) - w) * a * fast_rcp(lambda + a);
+            return (T(1) - wl) * c;
+        };
+        const T p1 = limited(k120 + k102, R.w3), p2 = limited(k210 + k012, R.w3), p3 = limited(k201 + k021, R.w3);
+        const T m1 = limited(k120 - k102, R.w4), m2 = limited(k210 - k012, R.w4), m3 = limited(k201 - k021, R.w4);
+        s120 = T(0.5) * (m1 + p1); s102 = T(0.5) * (p1 - m1);
+        s210 = T(0.5) * (m2 + p2); s012 = T(0.5) * (p2 - m2);
+        s201 = T(0.5) * (m3 + p3); s021 = T(0.5) * (p3 - m3);
+        s111 = limited(k111, R.w5);
+        const T visc = (T(1) / w1 - T(0.5)) * rho;
+        const T a4 = T(2) / T(3) * visc * R.A;
+        const T e43 = a4 * (Dxu - T(2) * Dyv + Dzw);
+        const T e44 = a4 * (-T(2) * Dxu + Dyv + Dzw);
+        const T e45 = -T(2) * a4 * (Dxu + Dyv + Dzw);
+        c220 = (e43 + e44 + e45) * third;
+        c202 = (e45 - e43) * third;
+        c022 = (e45 - e44) * third;
+        const T b4 = -third * visc * R.B;
+        c211 = b4 * DywDzv;
+        c121 = b4 * DxwDzu;
+        c112 = b4 * DxvDyu;
+    }
+
+    // ---- post-collision central moments ----
+    const T q211 = c211 + ((s200 + third) * s011 + T(2) * s101 * s110) * rhoInv;
+    const T q121 = c121 + ((s020 + third) * s101 + T(2) * s110 * s011) * rhoInv;
+    const T q112 = c112 + ((s002 + third) * s110 + T(2) * s011 * s101) * rhoInv;
+    const T q220 = c220 + ((s020 * s200 + T(2) * s110 * s110 + (s200 + s020) * third) * rhoInv - dRhoNinth);
+    const T q022 = c022 + ((s002 * s020 + T(2) * s011 * s011 + (s002 + s020) * third) * rhoInv - dRhoNinth);
+    const T q202 = c202 + ((s200 * s002 + T(2) * s101 * s101 + (s200 + s002) * third) * rhoInv - dRhoNinth);
+    const T q122 = (s020 * s102 + s002 * s120 + T(4) * s011 * s111 + T(2) * (s110 * s012 + s101 * s021) + (s120 + s102) * third) * rhoInv;
+    const T q212 = (s002 * s210 + s200 * s012 + T(4) * s101 * s111 + T(2) * (s011 * s201 + s110 * s102) + (s210 + s012) * third) * rhoInv;
+    const T q221 = (s200 * s021 + s020 * s201 + T(4) * s110 * s111 + T(2) * (s101 * s120 + s011 * s210) + (s021 + s201) * third) * rhoInv;
+    const T r2 = rhoInv * rhoInv;
+    const T q222 = (T(4) * s111 * s111 + s200 * q022 + s020 * q202 + s002 * q220 +
+                    T(4) * (s011 * q211 + s101 * q121 + s110 * q112) + T(2) * (s120 * s102 + s210 * s012 + s201 * s021)) * rhoInv
+                 - (T(16) * s110 * s101 * s011 + T(4) * (s101 * s101 * s020 + s011 * s011 * s200 + s110 * s110 * s002) +
+                    T(2) * s200 * s020 * s002) * r2
+                 + (T(3) * (q022 + q202 + q220) + (s200 + s020 + s002)) * rhoInv * ninth
+                 - T(2) / T(3) * (T(2) * (s101 * s101 + s011 * s011 + s110 * s110) + (s002 * s020 + s002 * s200 + s020 * s200) +
+                                  (s002 + s020 + s200) * third) * r2
+                 - (dRho * dRho - dRho) * r2 * (T(1) / T(27));
+
+    // ---- back transform (first moments flip sign: momentum gains the force) ----
+    return CentralMoments<T>{dRho, -k100, s200, -k001, s101, s201, s002, s102, q202,
+                              -k010, s110, s210, s011, s111, q211, s012, q112, q212,
+                              s020, s120, q220, s021, q121, q221, q022, q122, q222};
+}
+
 // f[27] in/out (shifted populations).  MODE 0: K17 or K15 from R.k17 at run
 // time; 1: K17; 2: K15.
 template <class T, int MODE = 0>
@@ -223,89 +321,151 @@ __host__ __device__ __forceinline__ void collide(T (&f)[27], const Relax<T> &R)
     cm_forward(y_a21, y_b21, y_c21, ux, ux2, T(0), k021, k121, k221);
     cm_forward(y_a22, y_b22, y_c22, ux, ux2, ninth, k022, k122, k222);
     (void)k212; (void)k221; (void)k122; (void)k222;
-
-    // fourth-order cumulants relax to their equilibrium (rate 1): their
-    // pre-collision values, and the fourth-order moments, are not needed
     (void)k211; (void)k121; (void)k112; (void)k220; (void)k022; (void)k202;
-    const T dRhoNinth = dRho * rhoInv * ninth;
 
-    // ---- relaxation ----
-    const T w1 = R.w1;
-    const T hr = T(0.5) * rhoInv;
-    const T Dxu = -w1 * hr * (T(2) * k200 - k020 - k002) - hr * (k200 + k020 + k002 - dRho);
-    const T Dyv = Dxu + T(1.5) * w1 * rhoInv * (k200 - k020);
-    const T Dzw = Dxu + T(1.5) * w1 * rhoInv * (k200 - k002);
-    const T DxvDyu = -T(3) * w1 * rhoInv * k110;
-    const T DxwDzu = -T(3) * w1 * rhoInv * k101;
-    const T DywDzv = -T(3) * w1 * rhoInv * k011;
-
-    const T om1 = T(1) - w1;
-    const T s110 = om1 * k110, s101 = om1 * k101, s011 = om1 * k011;
-    const T g1 = T(3) * rho * (T(1) - T(0.5) * w1);
-    const T g2 = T(1.5) * rho;   // 3 rho (1 - omega2/2), omega2 = 1
-    const T e33 = om1 * (k200 - k020) - g1 * (ux2 * Dxu - uy2 * Dyv);
-    const T e34 = om1 * (k200 - k002) - g1 * (ux2 * Dxu - uz2 * Dzw);
-    const T e35 = dRho - g2 * (ux2 * Dxu + uy2 * Dyv + uz2 * Dzw);
-    const T s200 = (e33 + e34 + e35) * third;
-    const T s020 = (e34 - T(2) * e33 + e35) * third;
-    const T s002 = (e33 - T(2) * e34 + e35) * third;
-
-    T s120 = 0, s102 = 0, s210 = 0, s012 = 0, s201 = 0, s021 = 0, s111 = 0;
-    T c220 = 0, c202 = 0, c022 = 0, c211 = 0, c121 = 0, c112 = 0;
-    const bool k17 = MODE == 1 || (MODE == 0 && R.k17);
-    if (MODE != 2 && k17) {
-        const T lambda = R.lambda;
-        // limited relaxation: the rate tends to 1 where the cumulant is large compared to lambda
-        auto limited = [&](T c, T w) {
-            const T a = c < T(0) ? -c : c;
-            const T wl = w + (T(1) - w) * a * fast_rcp(lambda + a);
-            return (T(1) - wl) * c;
-        };
-        const T p1 = limited(k120 + k102, R.w3), p2 = limited(k210 + k012, R.w3), p3 = limited(k201 + k021, R.w3);
-        const T m1 = limited(k120 - k102, R.w4), m2 = limited(k210 - k012, R.w4), m3 = limited(k201 - k021, R.w4);
-        s120 = T(0.5) * (m1 + p1); s102 = T(0.5) * (p1 - m1);
-        s210 = T(0.5) * (m2 + p2); s012 = T(0.5) * (p2 - m2);
-        s201 = T(0.5) * (m3 + p3); s021 = T(0.5) * (p3 - m3);
-        s111 = limited(k111, R.w5);
-        const T visc = (T(1) / w1 - T(0.5)) * rho;
-        const T a4 = T(2) / T(3) * visc * R.A;
-        const T e43 = a4 * (Dxu - T(2) * Dyv + Dzw);
-        const T e44 = a4 * (-T(2) * Dxu + Dyv + Dzw);
-        const T e45 = -T(2) * a4 * (Dxu + Dyv + Dzw);
-        c220 = (e43 + e44 + e45) * third;
-        c202 = (e45 - e43) * third;
-        c022 = (e45 - e44) * third;
-        const T b4 = -third * visc * R.B;
-        c211 = b4 * DywDzv;
-        c121 = b4 * DxwDzu;
-        c112 = b4 * DxvDyu;
-    }
-
-    // ---- post-collision central moments ----
-    const T q211 = c211 + ((s200 + third) * s011 + T(2) * s101 * s110) * rhoInv;
-    const T q121 = c121 + ((s020 + third) * s101 + T(2) * s110 * s011) * rhoInv;
-    const T q112 = c112 + ((s002 + third) * s110 + T(2) * s011 * s101) * rhoInv;
-    const T q220 = c220 + ((s020 * s200 + T(2) * s110 * s110 + (s200 + s020) * third) * rhoInv - dRhoNinth);
-    const T q022 = c022 + ((s002 * s020 + T(2) * s011 * s011 + (s002 + s020) * third) * rhoInv - dRhoNinth);
-    const T q202 = c202 + ((s200 * s002 + T(2) * s101 * s101 + (s200 + s002) * third) * rhoInv - dRhoNinth);
-    const T q122 = (s020 * s102 + s002 * s120 + T(4) * s011 * s111 + T(2) * (s110 * s012 + s101 * s021) + (s120 + s102) * third) * rhoInv;
-    const T q212 = (s002 * s210 + s200 * s012 + T(4) * s101 * s111 + T(2) * (s011 * s201 + s110 * s102) + (s210 + s012) * third) * rhoInv;
-    const T q221 = (s200 * s021 + s020 * s201 + T(4) * s110 * s111 + T(2) * (s101 * s120 + s011 * s210) + (s021 + s201) * third) * rhoInv;
-    const T r2 = rhoInv * rhoInv;
-    const T q222 = (T(4) * s111 * s111 + s200 * q022 + s020 * q202 + s002 * q220 +
-                    T(4) * (s011 * q211 + s101 * q121 + s110 * q112) + T(2) * (s120 * s102 + s210 * s012 + s201 * s021)) * rhoInv
-                 - (T(16) * s110 * s101 * s011 + T(4) * (s101 * s101 * s020 + s011 * s011 * s200 + s110 * s110 * s002) +
-                    T(2) * s200 * s020 * s002) * r2
-                 + (T(3) * (q022 + q202 + q220) + (s200 + s020 + s002)) * rhoInv * ninth
-                 - T(2) / T(3) * (T(2) * (s101 * s101 + s011 * s011 + s110 * s110) + (s002 * s020 + s002 * s200 + s020 * s200) +
-                                  (s002 + s020 + s200) * third) * r2
-                 - (dRho * dRho - dRho) * r2 * (T(1) / T(27));
-
-    // ---- back transform (first moments flip sign: momentum gains the force) ----
-    const CentralMoments<T> M{dRho, -k100, s200, -k001, s101, s201, s002, s102, q202,
-                              -k010, s110, s210, s011, s111, q211, s012, q112, q212,
-                              s020, s120, q220, s021, q121, q221, q022, q122, q222};
+    const LowMoments<T> K{k100, k010, k001, k200, k020, k002, k110, k101, k011, k120, k102, k210, k012, k201, k021, k111};
+    const CentralMoments<T> M = relax_moments<T, MODE>(K, dRho, rho, rhoInv, ux2, uy2, uz2, R);
     from_central_moments(f, M, ux, uy, uz);
+}
+
+// The collision on 16-bit stores' deviations: population q is w_q (h_q + Theta_q),
+// Theta the equilibrium at rho = 1 and the store's reference velocity U, a
+// product over the axes.  Both transforms are linear, so they run on h alone:
+// * each three-point chain carries the weights' ratio 1 : 4 : 1 (one fma in place
+//   of an add), 1/216 waits for the moments, and the back transform's powers of
+//   two and 1/w meet in one factor per direction;
+// * Theta's central moments about u are products of (1, -v, v^2 + 1/3) with
+//   v = u - U; only the low-order ones are added going in, all are taken off
+//   going out.
+// Decoding and encoding every population (an fma with two scalars, of which an
+// instruction takes only one; a subtraction and a product) and 81 scalar
+// constants are gone.  Per step: 256x64x64 duct BF16 31.5 -> 27.2 us, 106^3
+// vortex FP16 34.0 -> 32.4, 256x128x128 sphere BF16 94.3 -> 91.7 and FP16 93.6
+// -> 92.1 (half of its waves also hold an open cell and run its condition: 861
+// vector instructions per wave, which fill the time).
+// s, d, k per (x, y) chain along z, 3 (cx + 1) + (cy + 1): h+ + h-, h+ - h-,
+// (h+ + h-) + 4 h0.
+template <int MODE>
+__device__ __forceinline__ void collide_deviations(const float (&s)[9], const float (&d)[9], const float (&k)[9],
+                                                   const float (&U)[3], const Relax<float> &R, float (&h)[27])
+{
+    constexpr float n = 1.f / 216.f, third = 1.f / 3.f, ninth = 1.f / 9.f, r27 = 1.f / 27.f;
+    auto quad = [](float m, float z, float p) { return __builtin_fmaf(4.f, z, p + m); };
+    // ---- density and momentum of h, velocity ----
+    const float X0 = quad(k[0], k[1], k[2]), X1 = quad(k[3], k[4], k[5]), X2 = quad(k[6], k[7], k[8]);
+    const float dRho = n * quad(X0, X1, X2);
+    const float jx = n * (X2 - X0);
+    const float jy = n * quad(k[2] - k[0], k[5] - k[3], k[8] - k[6]);
+    const float jz = n * quad(quad(d[0], d[1], d[2]), quad(d[3], d[4], d[5]), quad(d[6], d[7], d[8]));
+    const float rho = 1.f + dRho, rhoInv = fast_rcp(rho);
+    const float vx = __builtin_fmaf(-dRho, U[0], __builtin_fmaf(0.5f, R.gx, jx)) * rhoInv;
+    const float vy = __builtin_fmaf(-dRho, U[1], __builtin_fmaf(0.5f, R.gy, jy)) * rhoInv;
+    const float vz = __builtin_fmaf(-dRho, U[2], __builtin_fmaf(0.5f, R.gz, jz)) * rhoInv;
+    const float ux = vx + U[0], uy = vy + U[1], uz = vz + U[2];
+    const float ux2 = ux * ux, uy2 = uy * uy, uz2 = uz * uz;
+    const float tx = 2.f * ux, ty = 2.f * uy, tz = 2.f * uz;
+    // ---- forward transform: z, y, x ----
+    float z1[9], z2[9];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) {
+        z1[c] = __builtin_fmaf(-uz, k[c], d[c]);
+        z2[c] = __builtin_fmaf(uz2, k[c], __builtin_fmaf(-tz, d[c], s[c]));
+    }
+    // y[order in y][x] of the z orders 0, 1, 2
+    float y0[3][3], y1[3][3], y2[3][3];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+        auto chain = [&](float m, float z, float p, float (&o)[3][3]) {
+            const float a = p + m, b = p - m, c = __builtin_fmaf(4.f, z, a);
+            o[0][x] = c;
+            o[1][x] = __builtin_fmaf(-uy, c, b);
+            o[2][x] = __builtin_fmaf(uy2, c, __builtin_fmaf(-ty, b, a));
+        };
+        chain(k[3 * x], k[3 * x + 1], k[3 * x + 2], y0);
+        chain(z1[3 * x], z1[3 * x + 1], z1[3 * x + 2], y1);
+        chain(z2[3 * x], z2[3 * x + 1], z2[3 * x + 2], y2);
+    }
+    auto zeroth = [&](const float (&c)[3]) { return quad(c[0], c[1], c[2]); };
+    auto first = [&](const float (&c)[3]) { return __builtin_fmaf(-ux, quad(c[0], c[1], c[2]), c[2] - c[0]); };
+    auto second = [&](const float (&c)[3]) {
+        const float a = c[2] + c[0], b = c[2] - c[0];
+        return __builtin_fmaf(ux2, __builtin_fmaf(4.f, c[1], a), __builtin_fmaf(-tx, b, a));
+    };
+    const float vx2 = vx * vx, vy2 = vy * vy, vz2 = vz * vz;
+    const float px = vx2 + third, py = vy2 + third, pz = vz2 + third;
+    const float vxy = vx * vy, vxz = vx * vz, vyz = vy * vz;
+    LowMoments<float> K{};
+    // the first moments to rounding, so that the collision keeps the momentum
+    K.k100 = __builtin_fmaf(-ux, dRho, jx) - vx;
+    K.k010 = __builtin_fmaf(-uy, dRho, jy) - vy;
+    K.k001 = __builtin_fmaf(-uz, dRho, jz) - vz;
+    K.k200 = __builtin_fmaf(n, second(y0[0]), vx2);
+    K.k020 = __builtin_fmaf(n, zeroth(y0[2]), vy2);
+    K.k002 = __builtin_fmaf(n, zeroth(y2[0]), vz2);
+    K.k110 = __builtin_fmaf(n, first(y0[1]), vxy);
+    K.k101 = __builtin_fmaf(n, first(y1[0]), vxz);
+    K.k011 = __builtin_fmaf(n, zeroth(y1[1]), vyz);
+    if constexpr (MODE != 2) {
+        K.k120 = __builtin_fmaf(n, first(y0[2]), -vx * py);
+        K.k102 = __builtin_fmaf(n, first(y2[0]), -vx * pz);
+        K.k210 = __builtin_fmaf(n, second(y0[1]), -vy * px);
+        K.k012 = __builtin_fmaf(n, zeroth(y2[1]), -vy * pz);
+        K.k201 = __builtin_fmaf(n, second(y1[0]), -vz * px);
+        K.k021 = __builtin_fmaf(n, zeroth(y1[2]), -vz * py);
+        K.k111 = __builtin_fmaf(n, first(y1[1]), -vxy * vz);
+    }
+    CentralMoments<float> M = relax_moments<float, MODE>(K, dRho, rho, rhoInv, ux2, uy2, uz2, R);
+    // ---- Theta's moments off ----
+    M.m100 += vx; M.m010 += vy; M.m001 += vz;
+    M.m200 -= vx2; M.m020 -= vy2; M.m002 -= vz2;
+    M.m110 -= vxy; M.m101 -= vxz; M.m011 -= vyz;
+    M.m120 = __builtin_fmaf(vx, py, M.m120); M.m102 = __builtin_fmaf(vx, pz, M.m102);
+    M.m210 = __builtin_fmaf(vy, px, M.m210); M.m012 = __builtin_fmaf(vy, pz, M.m012);
+    M.m201 = __builtin_fmaf(vz, px, M.m201); M.m021 = __builtin_fmaf(vz, py, M.m021);
+    M.m111 = __builtin_fmaf(vxy, vz, M.m111);
+    M.m211 = __builtin_fmaf(-px, vyz, M.m211); M.m121 = __builtin_fmaf(-py, vxz, M.m121); M.m112 = __builtin_fmaf(-pz, vxy, M.m112);
+    // p_a p_b - 1/9 and p_x p_y p_z - 1/27 without the constants' cancellation
+    const float exy = __builtin_fmaf(vx2, py, third * vy2), exz = __builtin_fmaf(vx2, pz, third * vz2);
+    const float eyz = __builtin_fmaf(vy2, pz, third * vz2);
+    M.m220 -= exy; M.m202 -= exz; M.m022 -= eyz;
+    const float pxy = exy + ninth, pxz = exz + ninth, pyz = eyz + ninth;
+    M.m122 = __builtin_fmaf(vx, pyz, M.m122); M.m212 = __builtin_fmaf(vy, pxz, M.m212); M.m221 = __builtin_fmaf(vz, pxy, M.m221);
+    M.m222 -= __builtin_fmaf(vx2, pyz, third * eyz);
+    (void)r27;
+    // ---- back transform: x, y, z; the outer two outputs doubled ----
+    auto back = [](float k0, float k1, float k2, float u, float t, float u2, float &m, float &z, float &p) {
+        const float S = __builtin_fmaf(k0, u2, __builtin_fmaf(t, k1, k2)), D = __builtin_fmaf(k0, u, k1);
+        m = S - D;
+        p = S + D;
+        z = k0 - S;
+    };
+    // b[x][y order][z order]
+    float b[3][3][3];
+    const float q[9][3] = {{dRho, M.m100, M.m200}, {M.m001, M.m101, M.m201}, {M.m002, M.m102, M.m202},
+                           {M.m010, M.m110, M.m210}, {M.m011, M.m111, M.m211}, {M.m012, M.m112, M.m212},
+                           {M.m020, M.m120, M.m220}, {M.m021, M.m121, M.m221}, {M.m022, M.m122, M.m222}};
+#pragma unroll
+    for (int c = 0; c < 9; ++c) back(q[c][0], q[c][1], q[c][2], ux, tx, ux2, b[0][c / 3][c % 3], b[1][c / 3][c % 3], b[2][c / 3][c % 3]);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+        float a[3][3];   // [y][z order]
+#pragma unroll
+        for (int o = 0; o < 3; ++o) back(b[x][0][o], b[x][1][o], b[x][2][o], uy, ty, uy2, a[0][o], a[1][o], a[2][o]);
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+            float m, z, p;
+            back(a[y][0], a[y][1], a[y][2], uz, tz, uz2, m, z, p);
+            // 1 / (2^axes w) of the directions (x, y, -1), (x, y, 0), (x, y, 1)
+            constexpr float f[4] = {3.375f, 6.75f, 13.5f, 27.f};
+            const int e = (x != 1) + (y != 1);
+            constexpr int dirs[3][3][3] = {{{MMM, MMO, MMP}, {MOM, MOO, MOP}, {MPM, MPO, MPP}},
+                                           {{OMM, OMO, OMP}, {OOM, OOO, OOP}, {OPM, OPO, OPP}},
+                                           {{PMM, PMO, PMP}, {POM, POO, POP}, {PPM, PPO, PPP}}};
+            h[dirs[x][y][0]] = f[e + 1] * m;
+            h[dirs[x][y][1]] = f[e] * z;
+            h[dirs[x][y][2]] = f[e + 1] * p;
+        }
+    }
 }
 
 // getDRhoUxUyUz (cellFunctions.h:257-279): density deviation and velocity

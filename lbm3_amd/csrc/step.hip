@@ -367,6 +367,65 @@ template <class S, class Off> __device__ __forceinline__ Off slot_offset(int cel
     return (Off(uint32_t(cell) / LBM3_TILE) * Off(27 * LBM3_TILE) + Off(uint32_t(cell) % LBM3_TILE)) * Off(sizeof(S));
 }
 
+// The bulk cell of 16-bit storage, on the stored deviations (collide_deviations):
+// raw loads, the chains' sums, collision, rounding, raw stores.  A wave holding an
+// open cell whose condition is pending takes the values as floats first, the
+// open lanes through their populations; the others never decode.
+template <class S, bool FLIP, int BULK, bool OPEN>
+__device__ __forceinline__ void deviation_cell(const StepArgs<S> &a, int iter, int cell, bool open, __amdgpu_buffer_rsrc_t r, const uint32_t (&off)[8],
+                                               unsigned (&bits)[14])
+{
+    using Tr = StoreTraits<S>;
+    auto load = [&](unsigned (&in)[27], int base) {
+#pragma unroll
+        for (int q = 0; q < 27; ++q)
+            in[q] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, (int)off[pre_nb(q)],
+                                                                         base + pre_plane(q, FLIP) * LBM3_TILE * 2, 0);
+    };
+    constexpr int dirs[9][3] = {{MMM, MMO, MMP}, {MOM, MOO, MOP}, {MPM, MPO, MPP}, {OMM, OMO, OMP}, {OOM, OOO, OOP},
+                                {OPM, OPO, OPP}, {PMM, PMO, PMP}, {POM, POO, POP}, {PPM, PPO, PPP}};
+    float s[9], d[9], k[9];
+    // each path loads for itself: values loaded before the branch were spilled
+    // across the condition's code (sphere 256x128x128 254 us per step in FP16).
+    // The zero hides from the compiler that both paths start alike.
+    if (OPEN && __ballot(open)) {
+        unsigned in[27];
+        int zero = 0;
+        __asm__("" : "+s"(zero));
+        load(in, zero);
+        float h[27];
+#pragma unroll
+        for (int q = 0; q < 27; ++q) h[q] = Tr::dev(in[q]);
+        if (open) {
+#pragma unroll
+            for (int q = 0; q < 27; ++q) h[q] = fmaf(h[q], weight<float>(q), a.cd.off[q]);
+            const int x = -(a.fast.cellRow[cell].x + 8);
+            open_dispatch<float>(h, x, a.open.meta[x], a.open.records, a.open.dRhoRef, a.open.uNormalRef, a.open.dRhoCum,
+                                 a.open.uNormalCum, iter, a.open.scale);
+#pragma unroll
+            for (int q = 0; q < 27; ++q) h[q] = (h[q] - a.cd.off[q]) * (1.f / weight<float>(q));
+        }
+#pragma unroll
+        for (int c = 0; c < 9; ++c) {
+            const float m = h[dirs[c][0]], p = h[dirs[c][2]];
+            s[c] = p + m;
+            d[c] = p - m;
+            k[c] = __builtin_fmaf(4.f, h[dirs[c][1]], s[c]);
+        }
+    } else {
+        unsigned in[27];
+        load(in, 0);
+#pragma unroll
+        for (int c = 0; c < 9; ++c) Tr::chain(in[dirs[c][0]], in[dirs[c][1]], in[dirs[c][2]], s[c], d[c], k[c]);
+    }
+    float h[27];
+    collide_deviations<BULK>(s, d, k, a.cd.u, relax_of<float>(a.bulk), h);
+#pragma unroll
+    for (int q = 0; q < 14; ++q) bits[q] = Tr::dev_bits2(h[2 * q < 27 ? 2 * q : 26], h[2 * q + 1 < 27 ? 2 * q + 1 : 26]);
+}
+
+__device__ __forceinline__ short half_of(const unsigned (&bits)[14], int q) { return (short)(q & 1 ? bits[q / 2] >> 16 : bits[q / 2]); }
+
 // IMG: a periodic ghost holds its source cell's populations, so it collides to
 // the same values and streams them into the cells beside it.  The source's
 // thread does that for it: after its own stores it writes its post-collision
@@ -410,6 +469,28 @@ __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell)
     if constexpr (sizeof(Off) == 4 && (sizeof(S) >= 4 || LBM3_BUF16 > 0)) {
         // raw buffer accesses: the plane offset is a scalar operand
         const __amdgpu_buffer_rsrc_t r = pop_rsrc(a.f, 27LL * padded_cells(a.fast.N) * (long long)sizeof(S));
+        if constexpr (sizeof(S) == 2 && !ROTOR) {
+            unsigned bits[14];
+            bool open = false;
+            if constexpr (OPEN) open = (a.param ? a.param->pending : a.open.pending) && mask_bit<ROT>(a.fast.openBits, cell);
+            deviation_cell<S, FLIP, BULK, OPEN>(a, a.param ? a.param->iter : a.open.iter, cell, open, r, off, bits);
+#pragma unroll
+            for (int q = 0; q < 27; ++q)
+                __builtin_amdgcn_raw_buffer_store_b16(half_of(bits, q), r, (int)off[post_nb(q)], post_plane(q, FLIP) * LBM3_TILE * 2, 0);
+            if constexpr (IMG)
+                for (; img >= 0;) {
+                    const int2 gi = a.fast.images.info[img];
+                    const int4 g0 = a.fast.images.nb[2 * (size_t)img], g1 = a.fast.images.nb[2 * (size_t)img + 1];
+                    const int gn[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+#pragma unroll
+                    for (int q = 1; q < 27; ++q)
+                        if ((gi.x >> q) & 1)
+                            __builtin_amdgcn_raw_buffer_store_b16(half_of(bits, q), r, (int)slot_offset<S, Off>(gn[post_nb(q)]),
+                                                                  post_plane(q, FLIP) * LBM3_TILE * 2, 0);
+                    img = gi.y;
+                }
+            return;
+        }
 #pragma unroll
         for (int q = 0; q < 27; ++q)
             f[q] = StoreTraits<S>::bload(r, off[pre_nb(q)], pre_plane(q, FLIP) * LBM3_TILE * int(sizeof(S)), q, a.cd);
@@ -504,6 +585,15 @@ __global__ __launch_bounds__(256) void k_open_groups(StepArgs<S> a)
     for (int k = 0; k < 8; ++k)
         off[k] = ((uint32_t(nb[k]) / LBM3_TILE) * uint32_t(27 * LBM3_TILE) + uint32_t(nb[k]) % LBM3_TILE) * uint32_t(sizeof(S));
     const __amdgpu_buffer_rsrc_t r = pop_rsrc(a.f, 27LL * padded_cells(a.fast.N) * (long long)sizeof(S));
+    if constexpr (sizeof(S) == 2) {
+        unsigned bits[14];
+        deviation_cell<S, FLIP, BULK, true>(a, a.param ? a.param->iter : a.open.iter, cell,
+                                            code <= -8 && (a.param ? a.param->pending : a.open.pending), r, off, bits);
+#pragma unroll
+        for (int q = 0; q < 27; ++q)
+            __builtin_amdgcn_raw_buffer_store_b16(half_of(bits, q), r, (int)off[post_nb(q)], post_plane(q, FLIP) * LBM3_TILE * 2, 0);
+        return;
+    }
     T f[27];
 #pragma unroll
     for (int q = 0; q < 27; ++q)

@@ -100,6 +100,7 @@ struct Codec {
     float off[27];
     float w[27];
     float iw[27];
+    float u[3];     // the reference velocity
 };
 
 // Raw buffer access for levels below 4 GiB: a wave-uniform buffer resource for
@@ -178,6 +179,33 @@ __device__ __forceinline__ unsigned short f16_bits(float y)
 }
 __device__ __forceinline__ float f16_value(unsigned short bits) { return __half2float(__ushort_as_half(bits)); }
 
+// The bulk kernel works on the stored deviations themselves (collide_deviations)
+// and converts without the codec's weights and offsets: `dev` is the value of
+// the stored bits, `dev_bits2` the bits of two values (low and high half).
+// FP16 sums and differences of two stored values take one v_fma_mix_f32, whose
+// operands may be halves: no conversion at all on the way in.
+__device__ __forceinline__ float f16_sum(unsigned a, unsigned b)
+{
+    float r;
+    __asm__("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,1]" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float f16_difference(unsigned a, unsigned b)
+{
+    float r;
+    __asm__("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float f16_times4_plus(unsigned a, float b)
+{
+    float r;
+    __asm__("v_fma_mix_f32 %0, %1, 4.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
 template <> struct StoreTraits<__half> {
     using compute = float;
     static __device__ __forceinline__ float load(const __half *p, int q, const Codec &c)
@@ -198,6 +226,19 @@ template <> struct StoreTraits<__half> {
     static __device__ __forceinline__ void bstore(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff, float v, int q, const Codec &c)
     {
         __builtin_amdgcn_raw_buffer_store_b16((short)f16_bits((v - c.off[q]) * c.iw[q]), r, (int)voff, soff, 0);
+    }
+    static __device__ __forceinline__ float dev(unsigned bits) { return f16_value((unsigned short)bits); }
+    static __device__ __forceinline__ unsigned dev_bits2(float x, float y)
+    {
+        // the products behind x and y stay apart from the conversion (f16_bits)
+        __asm__ volatile("" : "+v"(x), "+v"(y));
+        return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x, y}, f16x2));
+    }
+    static __device__ __forceinline__ void chain(unsigned m, unsigned z, unsigned p, float &s, float &d, float &k)
+    {
+        s = f16_sum(p, m);
+        d = f16_difference(p, m);
+        k = f16_times4_plus(z, s);
     }
 };
 
@@ -249,6 +290,18 @@ template <> struct StoreTraits<f16c> {
     {
         __builtin_amdgcn_raw_buffer_store_b16((short)f16c_encode((v - c.off[q]) * c.iw[q]), r, (int)voff, soff, 0);
     }
+    static __device__ __forceinline__ float dev(unsigned bits) { return f16c_decode(bits) * 0x1p112f; }
+    static __device__ __forceinline__ unsigned dev_bits2(float x, float y)
+    {
+        return (unsigned)f16c_encode(x * 0x1p-112f) | ((unsigned)f16c_encode(y * 0x1p-112f) << 16);
+    }
+    static __device__ __forceinline__ void chain(unsigned m, unsigned z, unsigned p, float &s, float &d, float &k)
+    {
+        const float fm = dev(m), fp = dev(p);
+        s = fp + fm;
+        d = fp - fm;
+        k = __builtin_fmaf(dev(z), 4.f, s);
+    }
 };
 
 template <> struct StoreTraits<__hip_bfloat16> {
@@ -276,6 +329,18 @@ template <> struct StoreTraits<__hip_bfloat16> {
         unsigned int u = __float_as_uint((v - c.off[q]) * c.iw[q]);
         u += 0x7FFFu + ((u >> 16) & 1u);
         __builtin_amdgcn_raw_buffer_store_b16((short)(unsigned short)(u >> 16), r, (int)voff, soff, 0);
+    }
+    static __device__ __forceinline__ float dev(unsigned bits) { return __uint_as_float(bits << 16); }
+    static __device__ __forceinline__ unsigned dev_bits2(float x, float y)
+    {
+        return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x, y}, bf16x2));
+    }
+    static __device__ __forceinline__ void chain(unsigned m, unsigned z, unsigned p, float &s, float &d, float &k)
+    {
+        const float fm = dev(m), fp = dev(p);
+        s = fp + fm;
+        d = fp - fm;
+        k = __builtin_fmaf(dev(z), 4.f, s);
     }
 };
 
