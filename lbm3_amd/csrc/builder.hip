@@ -1833,7 +1833,7 @@ int gpu_build(Sim &sim, const float *tri, const int *triCounts, int nBodies, lbm
             BCHK(hipMemcpyAsync(mm.p, init, sizeof(init), hipMemcpyHostToDevice, s));
             int *m = mm.p;
             const int *I = B.i.p, *J = B.j.p, *K = B.k.p;
-            hipLaunchKernelGGL(k_extent, dim3((unsigned)std::min<long long>(1024, (n + 255) / 256)), dim3(256), 0, s, (long long)n,
+            hipLaunchKernelGGL(k_extent, dim3((unsigned)std::min<long long>(64, (n + 255) / 256)), dim3(256), 0, s, (long long)n,
                                I, J, K, m);
             int h[6];
             BCHK(hipMemcpyAsync(h, mm.p, sizeof(h), hipMemcpyDeviceToHost, s));

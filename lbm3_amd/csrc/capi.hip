@@ -122,7 +122,10 @@ static int setup_local_bc(Sim &s, int level)
 
 static int settle_open(Sim &s, int L);
 
-// entry points of casehooks.hip into this file
+static int prepare_open_fusion(Sim &s, int L);
+
+// entry points of casehooks.hip and serve.hip into this file
+int prepare_cells(Sim &s, int level) { return prepare_open_fusion(s, level); }   // serve.hip
 int upload_open_records_of(Sim &s, Level &l) { return upload_open_records(s, l); }
 int settle_open_level(Sim &s, int level) { return settle_open(s, level); }
 int setup_local_bc_of(Sim &s, int level) { return setup_local_bc(s, level); }
@@ -558,10 +561,7 @@ template <class S> static void step_level(Sim &s, int level)
     // takes the ghosts as they are: a caller may have written them.  A captured
     // step keeps the copy, so that every replay is the same.
     const bool images = l.imagesReady && !slot;
-    if (images && l.ghostsStale) {
-        a.fast.skip = l.ghostSkip.p;
-        a.fast.images = {l.imageSources.p, l.imageHead.p, l.imageInfo.p, l.imageNb.p};
-    }
+    if (images && l.ghostsStale) a.fast.images = images_of(l);
     // side-stream choice 3: the wall-adjacent cells in blocks ahead of the bulk
     // blocks of one launch (not with rotated lanes or 64-bit offsets)
     const bool walls = overlap == 3 && l.W > 0 && !a.laneRot && !wide_level<S>(l.N);

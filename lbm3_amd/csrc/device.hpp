@@ -48,6 +48,7 @@ struct PeriodicImages {
     const int *head;           // [N] first ghost entry of a source cell
     const int2 *info;          // per ghost entry {directions another cell reads, next entry of the same source or -1}
     const int4 *nb;            // [2] per ghost entry: the ghost's eight neighbour cells
+    const uint64_t *skip;      // FastTopo::skip with the ghosts' bits set
 };
 
 struct FastTopo {
@@ -59,7 +60,7 @@ struct FastTopo {
     int nRows;
     const uint64_t *openBits;  // as skip: open cells the bulk kernel completes and steps itself; null: none
     const uint64_t *rotorBits; // as skip: cells the rotors can reach, stepped by the bulk kernel; null: none
-    PeriodicImages images;     // the periodic ghosts are stepped by their source cells (skip then covers them)
+    PeriodicImages images;     // the periodic ghosts are stepped by their source cells
 };
 
 constexpr int kRowPad = 4;

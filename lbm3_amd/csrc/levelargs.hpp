@@ -9,6 +9,11 @@ inline Topology topo_of(const Level &l)
     return Topology{l.N, l.shifter.p, l.ri.p, l.rj.p, l.rk.p, l.rjp.p, l.rkp.p, l.rjkp.p};
 }
 
+inline PeriodicImages images_of(const Level &l)
+{
+    return {l.imageSources.p, l.imageHead.p, l.imageInfo.p, l.imageNb.p, l.ghostSkip.p};
+}
+
 template <class S> inline StepArgs<S> step_args(Sim &s, Level &l)
 {
     StepArgs<S> a;

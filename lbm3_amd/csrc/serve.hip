@@ -4,9 +4,9 @@
 //
 // Requests queue on submit; every lbm3_server_step admits queued requests
 // while the HBM budget and the slot count allow (building their grids on the
-// GPU), advances every active request by one time step with four launches for
-// all of them together (bulk, wall-adjacent, open boundary, periodic copy:
-// k_multi_*), and retires the requests that reached their step count.  A
+// GPU), advances every active request by one time step with one launch per
+// storage type for all of them together (k_multi_step, and passes after it for
+// requests whose open boundary or ghosts need them), and retires the requests that reached their step count.  A
 // request admitted while others run joins the next batched step, so work of
 // requests that arrived at different times overlaps on the device.  Each
 // domain keeps its own esotwist parity, collision variant and boundary tables;
@@ -49,6 +49,7 @@ struct Request {
     long long estBytes = 0;
     double tSubmit = 0, tStart = 0, tFinish = 0;
     lbm3_sim *sim = nullptr;
+    int tick0 = 0;                       // the server's tick of its first step
     int done = 0;
     bool finished = false;
     int status = 0;                      // 0 ok, < 0: the LBM3_E_* code the request failed with
@@ -76,7 +77,10 @@ struct Server {
     std::vector<Request *> active;
     std::map<long long, std::unique_ptr<Request>> all;
     hipStream_t stream = nullptr;
-    DBuf<unsigned char> desc[5];      // device descriptors and block prefixes, one per storage type
+    DBuf<unsigned char> desc[5];      // device descriptors and block tables, one per storage type
+    bool stale[5] = {true, true, true, true, true};   // the active requests of the type changed since the upload
+    int blocks[5][4] = {};            // bulk, wall, open and periodic blocks of the uploaded tables
+    size_t tables[5] = {};            // offset of the tables behind the descriptors
     Stage stage[8];
     int nextStage = 0;
     long long stepsRun = 0, updatesRun = 0;
@@ -111,6 +115,8 @@ static long long estimate_bytes(const Request &r)
     return (long long)(cells * (27.0 * (double)storage_bytes(r.storage) + 64.0)) + (64LL << 20);
 }
 
+int prepare_cells(Sim &s, int level);     // capi.hip
+
 static int admit(Server &sv, Request &r)
 {
     int rc = lbm3_sim_create(&r.c, r.storage, &r.sim);
@@ -119,6 +125,13 @@ static int admit(Server &sv, Request &r)
                                    (int)r.counts.size(), r.dom, &updates);
     if (!rc && wide_level<double>(r.sim->s.L[0].N)) rc = set_error(LBM3_E_MEMORY, "request too large for the batched kernels");
     if (!rc) rc = lbm3_apply_initial_condition(r.sim, 0);
+    if (!rc) {
+        // the batched launch completes and steps the open cells and the ghosts itself where it can
+        Sim &s = r.sim->s;
+        s.tuneChosen = true;
+        s.tune.openGroup = 1;
+        rc = prepare_cells(s, 0);
+    }
     if (!rc) rc = check_hip(hipStreamSynchronize(r.sim->s.stream), "request build");
     if (rc) {
         if (r.sim) lbm3_sim_destroy(r.sim);
@@ -128,11 +141,7 @@ static int admit(Server &sv, Request &r)
         r.tStart = r.tFinish = now_s();
         return rc;
     }
-    // batched steps run the boundary condition as its own pass after streaming
-    Level &l = r.sim->s.L[0];
-    l.openFusionChecked = true;
-    l.fusedOpen = false;
-    l.openSettled = true;
+    sv.stale[r.storage] = true;
     r.fluidUpdates = updates;
     r.tStart = now_s();
     sv.used += r.estBytes;
@@ -158,33 +167,57 @@ static void retire(Server &sv, Request &r)
     sv.used -= r.estBytes;
 }
 
-template <class S> static int batched_step(Server &sv, int kind, const std::vector<Request *> &group)
+// descriptors and block tables of the active requests of one storage type
+template <class S> static int upload_domains(Server &sv, int kind, const std::vector<Request *> &group)
 {
     const int n = (int)group.size();
-    if (!n) return 0;
-    std::vector<MultiDesc<S>> D(n);
-    std::vector<int> st(4 * (size_t)(n + 1));
-    int blocks[4] = {0, 0, 0, 0};
+    std::vector<MultiDesc<S>> D((size_t)n);
+    std::vector<int> domain[2], start[2];   // bulk and wall blocks; open and periodic prefixes
     for (int d = 0; d < n; ++d) {
         Sim &s = group[d]->sim->s;
         Level &l = s.L[0];
         MultiDesc<S> &m = D[d];
+        if (group[d]->done == 0) group[d]->tick0 = (int)sv.stepsRun;
         m.step = step_args<S>(s, l);
+        m.open = open_args<S>(s, l, 0);
         m.step.open = FusedOpen<typename StoreTraits<S>::compute>{};
-        m.open = open_args<S>(s, l, l.info.iterationsFinished);
+        m.step.open.meta = m.open.meta;
+        m.step.open.records = m.open.records;
+        m.step.open.dRhoRef = m.open.dRhoRef;
+        m.step.open.uNormalRef = m.open.uNormalRef;
+        m.step.open.dRhoCum = m.open.dRhoCum;
+        m.step.open.uNormalCum = m.open.uNormalCum;
+        m.step.open.scale = m.open.scale;
+        m.step.fast.images = images_of(l);
         m.perIndex = l.perIndex.p;
         m.perSource = l.perSource.p;
         m.nPeriodic = l.nPeriodic;
-        m.flip = l.info.esotwistFlipper;
+        // the request's first tick and its state then
+        m.tick0 = group[d]->tick0;
+        m.iter0 = l.info.iterationsFinished - group[d]->done;
+        m.flip0 = (l.info.esotwistFlipper + group[d]->done) & 1;
         m.k17 = relax_of<typename StoreTraits<S>::compute>(l.bulk).k17;
-        const int per[4] = {(l.N + 255) / 256, (l.W + 255) / 256, (l.nOpen + 255) / 256, (l.nPeriodic + 255) / 256};
-        for (int k = 0; k < 4; ++k) {
-            st[(size_t)k * (n + 1) + d] = blocks[k];
-            blocks[k] += per[k];
+        m.fused = l.fusedOpen ? 1 : 0;
+        m.images = l.imagesReady ? 1 : 0;
+        m.bulkStart = (int)domain[0].size();
+        m.wallStart = (int)domain[1].size();
+        domain[0].insert(domain[0].end(), (size_t)((l.N + 255) / 256), d);
+        domain[1].insert(domain[1].end(), (size_t)((l.W + 255) / 256), d);
+        const int per[2] = {m.fused ? 0 : (l.nOpen + 255) / 256, m.images ? 0 : (l.nPeriodic + 255) / 256};
+        for (int k = 0; k < 2; ++k) {
+            if (d == 0) start[k].push_back(0);
+            start[k].push_back(start[k].back() + per[k]);
         }
     }
-    for (int k = 0; k < 4; ++k) st[(size_t)k * (n + 1) + n] = blocks[k];
-    // one upload of [descriptors | block prefixes] into this storage type's device buffer
+    int (&blocks)[4] = sv.blocks[kind];
+    for (int k = 0; k < 2; ++k) {
+        blocks[k] = (int)domain[k].size();
+        blocks[2 + k] = start[k].back();
+    }
+    // one upload of [descriptors | wall and bulk blocks' domains | prefixes]
+    std::vector<int> st(domain[1]);
+    st.insert(st.end(), domain[0].begin(), domain[0].end());
+    for (int k = 0; k < 2; ++k) st.insert(st.end(), start[k].begin(), start[k].end());
     const size_t db = (sizeof(MultiDesc<S>) * (size_t)n + 255) & ~size_t(255), sb = sizeof(int) * st.size();
     DBuf<unsigned char> &dev = sv.desc[kind];
     if ((size_t)dev.n < db + sb) {
@@ -198,14 +231,28 @@ template <class S> static int batched_step(Server &sv, int kind, const std::vect
     HIPCHK_RET(hipMemcpyAsync(dev.p, g->host, db + sb, hipMemcpyHostToDevice, sv.stream));
     HIPCHK_RET(hipEventRecord(g->done, sv.stream));
     g->pending = true;
-    launch_multi_step<S>(reinterpret_cast<const MultiDesc<S> *>(dev.p), reinterpret_cast<const int *>(dev.p + db), n,
-                         blocks, sv.stream);
+    sv.tables[kind] = db;
+    sv.stale[kind] = false;
+    return 0;
+}
+
+template <class S> static int batched_step(Server &sv, int kind, const std::vector<Request *> &group)
+{
+    const int n = (int)group.size();
+    if (!n) return 0;
+    if (sv.stale[kind])
+        if (const int rc = upload_domains<S>(sv, kind, group)) return rc;
+    const unsigned char *dev = sv.desc[kind].p;
+    launch_multi_step<S>(reinterpret_cast<const MultiDesc<S> *>(dev), reinterpret_cast<const int *>(dev + sv.tables[kind]), n,
+                         sv.blocks[kind], (int)sv.stepsRun, sv.stream);
     HIPCHK_RET(hipGetLastError());
     for (Request *r : group) {
         Level &l = r->sim->s.L[0];
         l.info.esotwistFlipper = l.info.esotwistFlipper ? 0 : 1;
         l.info.iterationsFinished++;
         l.info.iterationsSinceTrackerReset++;
+        if (l.fusedOpen) l.openSettled = false;
+        if (l.imagesReady) l.ghostsStale = true;
         r->done++;
         sv.updatesRun += r->fluidUpdates;
     }
@@ -314,6 +361,7 @@ int lbm3_server_step(lbm3_server *h, long long *completed, int cap, int *nComple
     std::vector<Request *> still;
     for (Request *r : sv.active) {
         if (r->done >= r->steps) {
+            sv.stale[r->storage] = true;
             retire(sv, *r);
             report(r);
         } else {

@@ -50,18 +50,23 @@ template <class S> void launch_open_cells(const StepArgs<S> &a, bool flip, hipSt
 template <class S> void launch_rotor_cells(const StepArgs<S> &a, bool flip, hipStream_t s);
 template <class S> void launch_collide_wall(const StepArgs<S> &a, bool flip, hipStream_t s);
 
-// one time step of many single-level domains in four launches (bulk, wall,
-// open boundary, periodic copy); starts holds four block-prefix arrays of n + 1
+// one time step (tick) of many single-level domains: one launch for the bulk,
+// wall-adjacent, open and ghost cells of all, and passes after it for the open
+// boundaries and periodic copies of the domains that need them.  blocks: bulk,
+// wall, open, periodic; tables: see launch_multi_step
 template <class S> struct MultiDesc {
     StepArgs<S> step;
-    OpenArgs<S> open;             // at the parity after this step
+    OpenArgs<S> open;
     const int *perIndex, *perSource;
     int nPeriodic;
-    int flip;                     // esotwist parity before this step
+    int tick0, flip0, iter0;      // the domain's first tick, its esotwist parity and finished iterations then
     int k17;                      // collision variant of the bulk cells
+    int fused;                    // the bulk blocks complete the open boundary
+    int images;                   // the bulk blocks step the ghosts (after the first tick)
+    int bulkStart, wallStart;     // first bulk and wall block
 };
 template <class S>
-void launch_multi_step(const MultiDesc<S> *D, const int *starts, int n, const int (&blocks)[4], hipStream_t s);
+void launch_multi_step(const MultiDesc<S> *D, const int *tables, int n, const int (&blocks)[4], int tick, hipStream_t s);
 template <class S> void launch_open(const OpenArgs<S> &a, bool flip, hipStream_t s);
 template <class S> void launch_periodic(S *f, const Topology &t, int count, const int *index, const int *source, bool flip, hipStream_t s);
 template <class S> void launch_init(S *f, const Topology &t, const InitDesc &d, const LevelGeom &g, const Codec &cd, bool flip,
