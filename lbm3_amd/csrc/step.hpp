@@ -86,6 +86,13 @@ template <class S> int launch_mass(const S *f, const Topology &t, const int *wal
                                    double divisor = 1.0, bool accumulate = false);
 void launch_wall_force(const double *gWall, int W, const uint32_t *wallData, const int *wallIndex, const Topology &t,
                        const LevelGeom &g, const double origin[3], int nBodies, double *partial, hipStream_t s);
+// blocks of launch_rotor_force for n marked rotor blocks, six partial sums each
+inline int rotor_force_blocks(int n)
+{
+    const long long b = (27LL * n + 255) / 256;
+    return (int)(b < 128 ? b : 128);
+}
+int launch_rotor_force(const RotorDev &d, const int *index, double *partial, hipStream_t s);
 template <class T> void launch_collide_batch(T *f, int n, const Relax<T> &R, hipStream_t s);
 void launch_open_nb(const Topology &t, int count, const int *cell, int4 *out, hipStream_t s);
 int launch_open_stats(const double *dRhoCum, const double *uNormalCum, const uint32_t *meta, int start, int count,
