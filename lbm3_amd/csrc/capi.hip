@@ -1486,8 +1486,13 @@ int lbm3_download_macros(lbm3_sim *h, int level, void *out)
     if (const int rc = settle_open(s, level)) return rc;
     Level &l = s.L[level];
     const size_t cb = compute_bytes(s.storage);
-    DBuf<unsigned char> d;
-    HIPCHK(d.alloc(4LL * l.N * (long long)cb));
+    // fields of up to 64 MiB are made in a buffer that the simulation keeps: an
+    // allocation and its release, which waits for the device, cost a 32^3 box
+    // more than the fields themselves
+    const long long bytes = 4LL * l.N * (long long)cb;
+    DBuf<unsigned char> own;
+    DBuf<unsigned char> &d = bytes <= (64LL << 20) ? s.fields : own;
+    if (d.n < bytes) HIPCHK(d.alloc(bytes));
     const bool flip = l.info.esotwistFlipper != 0;
     const Topology t = topo_of(l);
     switch (s.storage) {

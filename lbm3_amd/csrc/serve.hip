@@ -55,7 +55,8 @@ struct Request {
     int status = 0;                      // 0 ok, < 0: the LBM3_E_* code the request failed with
     long long fluidUpdates = 0;          // per step
     double kineticEnergy = 0, force[6] = {0, 0, 0, 0, 0, 0};
-    std::vector<unsigned char> macros;
+    std::unique_ptr<unsigned char[]> macros;   // left as allocated: the download fills it
+    size_t macrosBytes = 0;
 };
 
 } // namespace
@@ -157,8 +158,11 @@ static void retire(Server &sv, Request &r)
         (void)lbm3_wall_forces(r.sim, 0, origin, 1, r.force);
     }
     if (r.keepMacros) {
-        r.macros.resize(4 * (size_t)s.L[0].N * compute_bytes(r.storage));
-        (void)lbm3_download_macros(r.sim, 0, r.macros.data());
+        const size_t bytes = 4 * (size_t)s.L[0].N * compute_bytes(r.storage);
+        r.macros.reset(new (std::nothrow) unsigned char[bytes]);
+        if (!r.macros) r.status = set_error(LBM3_E_MEMORY, "host allocation");
+        else if (const int rc = lbm3_download_macros(r.sim, 0, r.macros.get())) r.status = rc;
+        else r.macrosBytes = bytes;
     }
     lbm3_sim_destroy(r.sim);
     r.sim = nullptr;
@@ -396,8 +400,8 @@ int lbm3_server_macros(lbm3_server *h, long long id, void *out, long long bytes)
     if (it == h->s.all.end()) return set_error(LBM3_E_ARG, "unknown request");
     const Request &r = *it->second;
     if (!r.finished || !r.keepMacros || r.status) return set_error(LBM3_E_STATE, "no macros kept for this request");
-    if (bytes < (long long)r.macros.size()) return set_error(LBM3_E_ARG, "buffer too small");
-    memcpy(out, r.macros.data(), r.macros.size());
+    if (bytes < (long long)r.macrosBytes) return set_error(LBM3_E_ARG, "buffer too small");
+    memcpy(out, r.macros.get(), r.macrosBytes);
     return 0;
 }
 

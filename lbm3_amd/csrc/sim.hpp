@@ -182,6 +182,7 @@ struct Sim {
     std::vector<StepParam> *dryRun = nullptr;
     DBuf<double> partial;            // reduction scratch
     DBuf<double> scalar;
+    DBuf<unsigned char> fields;      // lbm3_download_macros, up to 64 MiB
     int watchdog = 0;                // lbm3_run checks for non-finite populations every this many coarse steps (0: off)
     std::vector<std::vector<int>> stlEdges;   // shared-edge counts [3 T] of each static body of the last build
     // timing of the level-0 collide-stream launches

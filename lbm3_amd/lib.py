@@ -233,14 +233,14 @@ class Sim:
 
     def macros(self, level=0):
         n = self.info(level).cellCount
-        out = np.zeros((n, 4), np.float64 if self.storage == "f64" else np.float32)
+        out = np.empty((n, 4), np.float64 if self.storage == "f64" else np.float32)
         check(load().lbm3_download_macros(self.h, level, out.ctypes.data))
         return out
 
     def populations(self, level=0):
         n = self.info(level).cellCount
         dt = {"f32": np.float32, "f64": np.float64, "f16": np.float16, "bf16": np.uint16, "f16c": np.uint16}[self.storage]
-        out = np.zeros((27, n), dt)
+        out = np.empty((27, n), dt)
         check(load().lbm3_download_populations(self.h, level, out.ctypes.data, out.nbytes))
         return out
 
