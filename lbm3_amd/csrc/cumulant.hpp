@@ -81,38 +81,15 @@ __host__ __device__ __forceinline__ void cm_forward(T m, T z, T p, T u, T u2, T 
     k2 = s - T(2) * u * d + u2 * kk;
 }
 
-// the same for a chain whose weight moment is zero (x + 0 is not x to the
-// compiler, which keeps the sign of a zero)
-template <class T>
-__host__ __device__ __forceinline__ void cm_forward(T m, T z, T p, T u, T u2, T &k0, T &k1, T &k2)
-{
-    const T s = p + m, d = p - m;
-    k0 = s + z;
-    k1 = d - u * k0;
-    k2 = s - T(2) * u * d + u2 * k0;
-}
-
-// inverse of cm_forward, the outer two outputs doubled: their halves, one per
-// axis, meet in one factor per population at the end of the back transform (a
-// power of two: the same bits), 26 products instead of 54.  K is then the
-// weight moment times two per doubled axis.
+// inverse of cm_forward
 template <class T>
 __host__ __device__ __forceinline__ void cm_backward(T k0, T k1, T k2, T u, T u2, T K, T &m, T &z, T &p)
 {
     const T kk = k0 + K;
     const T S = kk * u2 + T(2) * u * k1 + k2;
     const T D = kk * u + k1;
-    m = S - D;
-    p = S + D;
-    z = k0 - S;
-}
-template <class T>
-__host__ __device__ __forceinline__ void cm_backward(T k0, T k1, T k2, T u, T u2, T &m, T &z, T &p)
-{
-    const T S = k0 * u2 + T(2) * u * k1 + k2;
-    const T D = k0 * u + k1;
-    m = S - D;
-    p = S + D;
+    m = T(0.5) * (S - D);
+    p = T(0.5) * (S + D);
     z = k0 - S;
 }
 
@@ -137,39 +114,37 @@ __host__ __device__ __forceinline__ void from_central_moments(T (&f)[27], const 
     T b_a10, b_b10, b_c10, b_a11, b_b11, b_c11, b_a12, b_b12, b_c12;
     T b_a20, b_b20, b_c20, b_a21, b_b21, b_c21, b_a22, b_b22, b_c22;
     cm_backward(M.m000, M.m100, M.m200, ux, ux2, T(1), b_a00, b_b00, b_c00);
-    cm_backward(M.m001, M.m101, M.m201, ux, ux2, b_a01, b_b01, b_c01);
+    cm_backward(M.m001, M.m101, M.m201, ux, ux2, T(0), b_a01, b_b01, b_c01);
     cm_backward(M.m002, M.m102, M.m202, ux, ux2, third, b_a02, b_b02, b_c02);
-    cm_backward(M.m010, M.m110, M.m210, ux, ux2, b_a10, b_b10, b_c10);
-    cm_backward(M.m011, M.m111, M.m211, ux, ux2, b_a11, b_b11, b_c11);
-    cm_backward(M.m012, M.m112, M.m212, ux, ux2, b_a12, b_b12, b_c12);
+    cm_backward(M.m010, M.m110, M.m210, ux, ux2, T(0), b_a10, b_b10, b_c10);
+    cm_backward(M.m011, M.m111, M.m211, ux, ux2, T(0), b_a11, b_b11, b_c11);
+    cm_backward(M.m012, M.m112, M.m212, ux, ux2, T(0), b_a12, b_b12, b_c12);
     cm_backward(M.m020, M.m120, M.m220, ux, ux2, third, b_a20, b_b20, b_c20);
-    cm_backward(M.m021, M.m121, M.m221, ux, ux2, b_a21, b_b21, b_c21);
+    cm_backward(M.m021, M.m121, M.m221, ux, ux2, T(0), b_a21, b_b21, b_c21);
     cm_backward(M.m022, M.m122, M.m222, ux, ux2, ninth, b_a22, b_b22, b_c22);
 
     T a_aa0, a_ab0, a_ac0, a_ba0, a_bb0, a_bc0, a_ca0, a_cb0, a_cc0;
     T a_aa1, a_ab1, a_ac1, a_ba1, a_bb1, a_bc1, a_ca1, a_cb1, a_cc1;
     T a_aa2, a_ab2, a_ac2, a_ba2, a_bb2, a_bc2, a_ca2, a_cb2, a_cc2;
-    cm_backward(b_a00, b_a10, b_a20, uy, uy2, T(2) * W6, a_aa0, a_ab0, a_ac0);
+    cm_backward(b_a00, b_a10, b_a20, uy, uy2, W6, a_aa0, a_ab0, a_ac0);
     cm_backward(b_b00, b_b10, b_b20, uy, uy2, W23, a_ba0, a_bb0, a_bc0);
-    cm_backward(b_c00, b_c10, b_c20, uy, uy2, T(2) * W6, a_ca0, a_cb0, a_cc0);
-    cm_backward(b_a01, b_a11, b_a21, uy, uy2, a_aa1, a_ab1, a_ac1);
-    cm_backward(b_b01, b_b11, b_b21, uy, uy2, a_ba1, a_bb1, a_bc1);
-    cm_backward(b_c01, b_c11, b_c21, uy, uy2, a_ca1, a_cb1, a_cc1);
-    cm_backward(b_a02, b_a12, b_a22, uy, uy2, T(2) * W18, a_aa2, a_ab2, a_ac2);
+    cm_backward(b_c00, b_c10, b_c20, uy, uy2, W6, a_ca0, a_cb0, a_cc0);
+    cm_backward(b_a01, b_a11, b_a21, uy, uy2, T(0), a_aa1, a_ab1, a_ac1);
+    cm_backward(b_b01, b_b11, b_b21, uy, uy2, T(0), a_ba1, a_bb1, a_bc1);
+    cm_backward(b_c01, b_c11, b_c21, uy, uy2, T(0), a_ca1, a_cb1, a_cc1);
+    cm_backward(b_a02, b_a12, b_a22, uy, uy2, W18, a_aa2, a_ab2, a_ac2);
     cm_backward(b_b02, b_b12, b_b22, uy, uy2, W29, a_ba2, a_bb2, a_bc2);
-    cm_backward(b_c02, b_c12, b_c22, uy, uy2, T(2) * W18, a_ca2, a_cb2, a_cc2);
+    cm_backward(b_c02, b_c12, b_c22, uy, uy2, W18, a_ca2, a_cb2, a_cc2);
 
-    cm_backward(a_aa0, a_aa1, a_aa2, uz, uz2, T(4) * W36, f[MMM], f[MMO], f[MMP]);
-    cm_backward(a_ab0, a_ab1, a_ab2, uz, uz2, T(2) * W9, f[MOM], f[MOO], f[MOP]);
-    cm_backward(a_ac0, a_ac1, a_ac2, uz, uz2, T(4) * W36, f[MPM], f[MPO], f[MPP]);
-    cm_backward(a_ba0, a_ba1, a_ba2, uz, uz2, T(2) * W9, f[OMM], f[OMO], f[OMP]);
+    cm_backward(a_aa0, a_aa1, a_aa2, uz, uz2, W36, f[MMM], f[MMO], f[MMP]);
+    cm_backward(a_ab0, a_ab1, a_ab2, uz, uz2, W9, f[MOM], f[MOO], f[MOP]);
+    cm_backward(a_ac0, a_ac1, a_ac2, uz, uz2, W36, f[MPM], f[MPO], f[MPP]);
+    cm_backward(a_ba0, a_ba1, a_ba2, uz, uz2, W9, f[OMM], f[OMO], f[OMP]);
     cm_backward(a_bb0, a_bb1, a_bb2, uz, uz2, W49, f[OOM], f[OOO], f[OOP]);
-    cm_backward(a_bc0, a_bc1, a_bc2, uz, uz2, T(2) * W9, f[OPM], f[OPO], f[OPP]);
-    cm_backward(a_ca0, a_ca1, a_ca2, uz, uz2, T(4) * W36, f[PMM], f[PMO], f[PMP]);
-    cm_backward(a_cb0, a_cb1, a_cb2, uz, uz2, T(2) * W9, f[POM], f[POO], f[POP]);
-    cm_backward(a_cc0, a_cc1, a_cc2, uz, uz2, T(4) * W36, f[PPM], f[PPO], f[PPP]);
-#pragma unroll
-    for (int q = 1; q < 27; ++q) f[q] *= q < 7 ? T(0.5) : q < 19 ? T(0.25) : T(0.125);
+    cm_backward(a_bc0, a_bc1, a_bc2, uz, uz2, W9, f[OPM], f[OPO], f[OPP]);
+    cm_backward(a_ca0, a_ca1, a_ca2, uz, uz2, W36, f[PMM], f[PMO], f[PMP]);
+    cm_backward(a_cb0, a_cb1, a_cb2, uz, uz2, W9, f[POM], f[POO], f[POP]);
+    cm_backward(a_cc0, a_cc1, a_cc2, uz, uz2, W36, f[PPM], f[PPO], f[PPP]);
 }
 
 // central moments up to third order (well-conditioned: the weights' own are taken off)
@@ -318,9 +293,9 @@ __host__ __device__ __forceinline__ void collide(T (&f)[27], const Relax<T> &R)
     cm_forward(z_aa0, z_ab0, z_ac0, uy, uy2, W6, y_a00, y_a10, y_a20);
     cm_forward(z_ba0, z_bb0, z_bc0, uy, uy2, W23, y_b00, y_b10, y_b20);
     cm_forward(z_ca0, z_cb0, z_cc0, uy, uy2, W6, y_c00, y_c10, y_c20);
-    cm_forward(z_aa1, z_ab1, z_ac1, uy, uy2, y_a01, y_a11, y_a21);
-    cm_forward(z_ba1, z_bb1, z_bc1, uy, uy2, y_b01, y_b11, y_b21);
-    cm_forward(z_ca1, z_cb1, z_cc1, uy, uy2, y_c01, y_c11, y_c21);
+    cm_forward(z_aa1, z_ab1, z_ac1, uy, uy2, T(0), y_a01, y_a11, y_a21);
+    cm_forward(z_ba1, z_bb1, z_bc1, uy, uy2, T(0), y_b01, y_b11, y_b21);
+    cm_forward(z_ca1, z_cb1, z_cc1, uy, uy2, T(0), y_c01, y_c11, y_c21);
     cm_forward(z_aa2, z_ab2, z_ac2, uy, uy2, W18, y_a02, y_a12, y_a22);
     cm_forward(z_ba2, z_bb2, z_bc2, uy, uy2, W29, y_b02, y_b12, y_b22);
     cm_forward(z_ca2, z_cb2, z_cc2, uy, uy2, W18, y_c02, y_c12, y_c22);
@@ -337,13 +312,13 @@ __host__ __device__ __forceinline__ void collide(T (&f)[27], const Relax<T> &R)
         k100 = d - ux * kk;
         k200 = s - T(2) * ux * d + ux2 * kk;
     }
-    cm_forward(y_a01, y_b01, y_c01, ux, ux2, k001, k101, k201);
+    cm_forward(y_a01, y_b01, y_c01, ux, ux2, T(0), k001, k101, k201);
     cm_forward(y_a02, y_b02, y_c02, ux, ux2, third, k002, k102, k202);
-    cm_forward(y_a10, y_b10, y_c10, ux, ux2, k010, k110, k210);
-    cm_forward(y_a11, y_b11, y_c11, ux, ux2, k011, k111, k211);
-    cm_forward(y_a12, y_b12, y_c12, ux, ux2, k012, k112, k212);
+    cm_forward(y_a10, y_b10, y_c10, ux, ux2, T(0), k010, k110, k210);
+    cm_forward(y_a11, y_b11, y_c11, ux, ux2, T(0), k011, k111, k211);
+    cm_forward(y_a12, y_b12, y_c12, ux, ux2, T(0), k012, k112, k212);
     cm_forward(y_a20, y_b20, y_c20, ux, ux2, third, k020, k120, k220);
-    cm_forward(y_a21, y_b21, y_c21, ux, ux2, k021, k121, k221);
+    cm_forward(y_a21, y_b21, y_c21, ux, ux2, T(0), k021, k121, k221);
     cm_forward(y_a22, y_b22, y_c22, ux, ux2, ninth, k022, k122, k222);
     (void)k212; (void)k221; (void)k122; (void)k222;
     (void)k211; (void)k121; (void)k112; (void)k220; (void)k022; (void)k202;
