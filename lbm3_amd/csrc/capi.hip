@@ -203,6 +203,10 @@ static bool wide_of(const Sim &s, const Level &l)
 //   always been reported as cells of a kernel of their own.
 // * the levels in order on one stream: three-level sphere 344, with a stream
 //   per level 384.
+// * wall cells on a side stream again on a refined level of more than 200 MiB,
+//   whose step runs at the copy rate: three states of a three-level sphere in
+//   turn 793 against 822 (finest level 333 MB, 88 cells across) and 619 / 687
+//   (250 MB, 80 across); 385 / 345 at 128 MB (64 across).
 // * block order: one contiguous part per XCD, swept backwards every other step
 //   (order 3), so that each XCD's L2 and the last-level cache still hold what
 //   the step starts on: 64^3 vortex 14.9 against 18.3 in plain order, duct
@@ -211,8 +215,9 @@ static bool wide_of(const Sim &s, const Level &l)
 //   (729 MB) 272 against 289, and where rotors make some parts slower than
 //   others: rotor duct 286 / 306.
 // * occupancy cap of the bulk kernel (40 KiB of LDS per block, four blocks per
-//   CU: their tiles then fit an XCD's L2): above 1 GiB, 400x200x200 632 against
-//   692 (300x150x150: 277 / 272), and on levels of 64 to 256 MiB without open
+//   CU: their tiles then fit an XCD's L2): above 512 MiB, 400x200x200 632
+//   against 692, three 300x150x150 states in turn 302 / 324, one alone the same
+//   within 2%; on the refined levels of more than 200 MiB; and on levels of 64 to 256 MiB without open
 //   cells, three-level sphere 344 / 354, 130^3 vortex 91.2 / 93.2 (50 MB level
 //   25.2 / 23.6, 158^3 vortex of 443 MB 154 / 147).  Never for 16-bit storage,
 //   whose kernels are bound by instructions: FP16 256x128x128 115 / 94,
@@ -223,12 +228,13 @@ Sim::Tune tune_of(const Sim &s, const Level &l)
     constexpr long long MiB = 1LL << 20;
     const long long size = (long long)storage_bytes(s.storage), bytes = 27 * size * l.N;
     Sim::Tune t;
-    t.overlap = 3;
+    const bool deep = s.levels > 1 && l.W > 0 && !l.openInBulk && l.rotors.empty() && bytes > 200 * MiB;
+    t.overlap = deep ? 1 : 3;
     t.ordered = true;
     t.rotorInBulk = 1;
     t.openGroup = l.N > 32768 ? 1 : 0;
     t.xcdRemap = !l.rotors.empty() || bytes > 512 * MiB ? 2 : 3;
-    const bool cap = bytes > 1024 * MiB || (!l.openInBulk && bytes > 64 * MiB && bytes <= 256 * MiB);
+    const bool cap = deep || bytes > 512 * MiB || (!l.openInBulk && bytes > 64 * MiB && bytes <= 256 * MiB);
     t.bulkLds = size >= 4 && cap ? LBM3_BULK_LDS : 0;
     return t;
 }
