@@ -23,6 +23,7 @@ int set_error(int code, const std::string &msg)
 int check_hip(hipError_t e, const char *what)
 {
     if (e == hipSuccess) return 0;
+    (void)hipGetLastError();   // reported here: the next launch's check must not find it again
     return set_error(LBM3_E_HIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 

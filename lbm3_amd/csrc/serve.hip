@@ -18,6 +18,7 @@
 #include <memory>
 #include <new>
 #include <vector>
+#include "batch.hpp"
 #include "sim.hpp"
 #include "levelargs.hpp"
 
@@ -49,7 +50,6 @@ struct Request {
     long long estBytes = 0;
     double tSubmit = 0, tStart = 0, tFinish = 0;
     lbm3_sim *sim = nullptr;
-    int tick0 = 0;                       // the server's tick of its first step
     int done = 0;
     bool finished = false;
     int status = 0;                      // 0 ok, < 0: the LBM3_E_* code the request failed with
@@ -79,7 +79,7 @@ struct Server {
     std::map<long long, std::unique_ptr<Request>> all;
     hipStream_t stream = nullptr;
     DBuf<unsigned char> desc[5];      // device descriptors and block tables, one per storage type
-    bool stale[5] = {true, true, true, true, true};   // the active requests of the type changed since the upload
+    Batch batch[5];                   // tick and upload state per storage type
     int blocks[5][4] = {};            // bulk, wall, open and periodic blocks of the uploaded tables
     size_t tables[5] = {};            // offset of the tables behind the descriptors
     Stage stage[8];
@@ -142,7 +142,7 @@ static int admit(Server &sv, Request &r)
         r.tStart = r.tFinish = now_s();
         return rc;
     }
-    sv.stale[r.storage] = true;
+    sv.batch[r.storage].stale = true;
     r.fluidUpdates = updates;
     r.tStart = now_s();
     sv.used += r.estBytes;
@@ -181,7 +181,6 @@ template <class S> static int upload_domains(Server &sv, int kind, const std::ve
         Sim &s = group[d]->sim->s;
         Level &l = s.L[0];
         MultiDesc<S> &m = D[d];
-        if (group[d]->done == 0) group[d]->tick0 = (int)sv.stepsRun;
         m.step = step_args<S>(s, l);
         m.open = open_args<S>(s, l, 0);
         m.step.open = FusedOpen<typename StoreTraits<S>::compute>{};
@@ -197,7 +196,7 @@ template <class S> static int upload_domains(Server &sv, int kind, const std::ve
         m.perSource = l.perSource.p;
         m.nPeriodic = l.nPeriodic;
         // the request's first tick and its state then
-        m.tick0 = group[d]->tick0;
+        m.tick0 = sv.batch[kind].tick - group[d]->done;
         m.iter0 = l.info.iterationsFinished - group[d]->done;
         m.flip0 = (l.info.esotwistFlipper + group[d]->done) & 1;
         m.k17 = relax_of<typename StoreTraits<S>::compute>(l.bulk).k17;
@@ -236,31 +235,28 @@ template <class S> static int upload_domains(Server &sv, int kind, const std::ve
     HIPCHK_RET(hipEventRecord(g->done, sv.stream));
     g->pending = true;
     sv.tables[kind] = db;
-    sv.stale[kind] = false;
     return 0;
 }
 
 template <class S> static int batched_step(Server &sv, int kind, const std::vector<Request *> &group)
 {
-    const int n = (int)group.size();
-    if (!n) return 0;
-    if (sv.stale[kind])
-        if (const int rc = upload_domains<S>(sv, kind, group)) return rc;
-    const unsigned char *dev = sv.desc[kind].p;
-    launch_multi_step<S>(reinterpret_cast<const MultiDesc<S> *>(dev), reinterpret_cast<const int *>(dev + sv.tables[kind]), n,
-                         sv.blocks[kind], (int)sv.stepsRun, sv.stream);
-    HIPCHK_RET(hipGetLastError());
-    for (Request *r : group) {
-        Level &l = r->sim->s.L[0];
-        l.info.esotwistFlipper = l.info.esotwistFlipper ? 0 : 1;
-        l.info.iterationsFinished++;
-        l.info.iterationsSinceTrackerReset++;
-        if (l.fusedOpen) l.openSettled = false;
-        if (l.imagesReady) l.ghostsStale = true;
-        r->done++;
-        sv.updatesRun += r->fluidUpdates;
-    }
-    return 0;
+    return step_batch(
+        sv.batch[kind], group, [&](const std::vector<Request *> &run) { return upload_domains<S>(sv, kind, run); },
+        [&](int n, int tick) {
+            const unsigned char *dev = sv.desc[kind].p;
+            launch_multi_step<S>(reinterpret_cast<const MultiDesc<S> *>(dev),
+                                 reinterpret_cast<const int *>(dev + sv.tables[kind]), n, sv.blocks[kind], tick, sv.stream);
+            return check_hip(hipGetLastError(), "batched step");
+        },
+        [&](Request *r) {
+            Level &l = r->sim->s.L[0];
+            l.info.esotwistFlipper = l.info.esotwistFlipper ? 0 : 1;
+            l.info.iterationsFinished++;
+            l.info.iterationsSinceTrackerReset++;
+            if (l.fusedOpen) l.openSettled = false;
+            if (l.imagesReady) l.ghostsStale = true;
+            sv.updatesRun += r->fluidUpdates;
+        });
 }
 
 } // namespace lbm3
@@ -365,7 +361,7 @@ int lbm3_server_step(lbm3_server *h, long long *completed, int cap, int *nComple
     std::vector<Request *> still;
     for (Request *r : sv.active) {
         if (r->done >= r->steps) {
-            sv.stale[r->storage] = true;
+            sv.batch[r->storage].stale = true;
             retire(sv, *r);
             report(r);
         } else {
