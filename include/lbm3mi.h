@@ -195,7 +195,9 @@ int lbm3_download_array(lbm3_sim *s, int level, const char *name, void *out, lon
  * simulation's own buffer (valid until the level is rebuilt or the sim is
  * destroyed), *count its element count.  "f" gives the populations (storage
  * type; tiled, see lbm3_population_layout), after any pending open-boundary
- * completion is applied.  Replaces the case files' direct view access
+ * completion is applied and the periodic ghost cells hold their sources' values;
+ * from then on every call that steps leaves the ghosts so and takes what the
+ * caller wrote there.  Replaces the case files' direct view access
  * (Grid.fArray.getConstView(), Grid.IJKNBR.*, Grid.Wall.*:
  * taylorGreenVortexMain.cu:142-155). */
 int lbm3_device_array(lbm3_sim *s, int level, const char *name, void **ptr, long long *count);

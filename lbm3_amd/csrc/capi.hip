@@ -152,6 +152,7 @@ int finish_level_setup(Sim &s, int level)
     l.openFusionChecked = false;
     l.imagesReady = false;
     l.ghostsStale = false;
+    l.shared = false;
     l.fusedOpen = false;
     l.openInBulk = false;
     l.rotorInBulk = false;
@@ -476,6 +477,17 @@ static int settle_ghosts(Sim &s, Level &l)
     default: periodic_typed<float>(s, l, flip); break;
     }
     return check_hip(hipGetLastError(), "periodic ghost copy");
+}
+
+// The end of every call that steps: a caller who holds a level's populations
+// (lbm3_device_array) finds the ghosts copied, as after every step before the
+// bulk kernel stepped them, and the next step takes what that caller wrote there.
+static int settle_shared(Sim &s)
+{
+    for (int L = 0; L < s.levels; ++L)
+        if (s.L[L].shared)
+            if (const int rc = settle_ghosts(s, s.L[L])) return rc;
+    return 0;
 }
 
 // A condition is pending after a fused step and after a checkpoint load that
@@ -1070,6 +1082,7 @@ int lbm3_update_single_grid(lbm3_sim *h, int level)
     if (!h->s.L[level].openFusionChecked)
         if (const int rc = prepare_open_fusion(h->s, level)) return rc;
     step_level_any(h->s, level);
+    if (const int rc = settle_shared(h->s)) return rc;
     return check_hip(hipGetLastError(), "updateSingleGrid launch");
 }
 
@@ -1078,6 +1091,7 @@ int lbm3_update_all_grids(lbm3_sim *h, int level)
     if (!h) return set_error(LBM3_E_ARG, "null sim");
     if (const int rc = check_run(h->s, level)) return rc;
     update_all(h->s, level);
+    if (const int rc = settle_shared(h->s)) return rc;
     return check_hip(hipGetLastError(), "updateAllGrids launch");
 }
 
@@ -1095,6 +1109,7 @@ int lbm3_run(lbm3_sim *h, int steps)
         if (s.watchdog > 0 && ((s.L[0].info.iterationsFinished % s.watchdog) == 0 || t == steps - 1))
             if (const int rc = finite_state(s)) return rc;
     }
+    if (const int rc = settle_shared(s)) return rc;
     return check_hip(hipGetLastError(), "run launch");
 }
 
@@ -1433,6 +1448,7 @@ int lbm3_run_graph(lbm3_sim *h, int steps)
         if (es != hipSuccess) return check_hip(es, "step graph replay");
     }
     if (steps % 2) update_all(s, 0);
+    if (const int rc = settle_shared(s)) return rc;
     return check_hip(hipGetLastError(), "graph run");
 }
 
@@ -1454,8 +1470,9 @@ int lbm3_run_timed(lbm3_sim *h, int steps, int kernelEvents, double *out)
     s.evUsed = 0;
     HIPCHK(hipEventRecord(a, s.stream));
     for (int t = 0; t < steps; ++t) update_all(s, 0);
-    HIPCHK(hipEventRecord(b, s.stream));
     s.timing = false;
+    if (const int rc = settle_shared(s)) return rc;
+    HIPCHK(hipEventRecord(b, s.stream));
     HIPCHK(hipEventSynchronize(b));
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, a, b));
@@ -1575,7 +1592,12 @@ int lbm3_device_array(lbm3_sim *h, int level, const char *name, void **ptr, long
     Level &l = s.L[level];
     if (!l.built) return set_error(LBM3_E_STATE, "level not built");
     if (!strcmp(name, "f")) {
+        // the ghost copy is waited for: a caller that synchronized after its run
+        // may read on a stream of its own at once
+        const bool wait = l.ghostsStale;
         if (const int rc = settle_open(s, level)) return rc;
+        if (wait) HIPCHK(hipStreamSynchronize(s.stream));
+        l.shared = true;
         *ptr = l.f.p;
         *count = 27LL * padded_cells(l.N);
         return 0;

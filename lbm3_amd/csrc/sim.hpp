@@ -77,6 +77,7 @@ struct Level {
     // the bulk kernel steps the periodic ghosts from their source cells (PeriodicImages)
     bool imagesReady = false;        // the tables below are made, for the current cell records
     bool ghostsStale = false;        // the ghosts' own populations lag behind their sources'
+    bool shared = false;             // a caller holds the populations' address: no call returns with stale ghosts
     DBuf<uint64_t> ghostSkip, imageSources;
     DBuf<int> imageHead;
     DBuf<int2> imageInfo;

@@ -1,6 +1,8 @@
 """Periodic ghosts stepped by their source cells (one launch per step) against
 the copy after every step, on the GPU: the same populations bit for bit.  A
 captured step (run_graph) keeps the copy, so a replayed run is the copy path."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -108,3 +110,60 @@ def test_default_choices_equal_the_side_stream_kernels(storage):
         assert (s.cell_kinds(0)["open_in_bulk"] > 0) == (chosen is None)
         out.append((s.populations(0).tobytes(), s.wall_forces(0).tobytes()))
     assert out[0] == out[1]
+
+
+class _Kept:
+    """The simulation's FP32 populations through their address (lbm3_device_array),
+    copied on a stream other than the simulation's."""
+
+    def __init__(self, s):
+        L = lib.load()
+        self.copy = L.hipMemcpy     # of the runtime the library itself uses
+        ptr, n, tile, size = ctypes.c_void_p(), ctypes.c_longlong(), ctypes.c_int(), ctypes.c_int()
+        lib.check(L.lbm3_device_array(s.h, 0, b"f", ctypes.byref(ptr), ctypes.byref(n)))
+        lib.check(L.lbm3_population_layout(s.h, ctypes.byref(tile), ctypes.byref(size)))
+        self.ptr, self.cells = ptr, s.info(0).cellCount
+        self.shape = (n.value // (27 * tile.value), 27, tile.value)
+
+    def _copy(self, dst, src, host, kind):
+        assert self.copy(dst, src, ctypes.c_size_t(host.nbytes), kind) == 0
+
+    def read(self):
+        t = np.empty(self.shape, np.float32)
+        self._copy(ctypes.c_void_p(t.ctypes.data), self.ptr, t, 2)
+        return np.ascontiguousarray(t.transpose(1, 0, 2).reshape(27, -1)[:, :self.cells])
+
+    def write(self, planes):
+        t = np.zeros((27, self.shape[0] * self.shape[2]), np.float32)
+        t[:, :self.cells] = planes
+        t = np.ascontiguousarray(t.reshape(27, self.shape[0], self.shape[2]).transpose(1, 0, 2))
+        self._copy(self.ptr, ctypes.c_void_p(t.ctypes.data), t, 1)
+
+
+@pytest.mark.parametrize("box", ["cube 14", "cube 30 K17", "cube 62"])
+def test_a_kept_address_sees_and_sets_the_ghosts(box):
+    """The populations' address taken once: whatever call stepped, the ghosts are
+    their sources' when it is waited for, and what is written there is what the
+    next step takes (a simulation that gets the same state by upload)."""
+    a, b = (_make(*BOXES[box](), "f32", 4) for _ in range(2))
+    a.run(4)
+    a.sync()
+    f = _Kept(a)
+    first = f.read()
+    b.run_graph(4)
+    assert first.tobytes() == b.populations(0).tobytes()
+    ghosts = a.array("periodicIndex", 0)
+    for k, step in enumerate((lambda s: s.run(3), lambda s: s.run_graph(5), lambda s: s.run_timed(2, kernel_events=False),
+                              lambda s: s.run(1))):
+        step(a)
+        a.sync()
+        now = f.read()
+        b.run_graph((3, 5, 2, 1)[k])
+        assert now.tobytes() == b.populations(0).tobytes(), k
+        # the ghosts get other values through the address
+        now[:, ghosts[::3]] *= np.float32(1.25)
+        f.write(now)
+        b.set_populations(0, now)
+    a.run(2)
+    b.run_graph(2)
+    assert a.populations(0).tobytes() == b.populations(0).tobytes()
