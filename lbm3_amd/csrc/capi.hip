@@ -200,9 +200,8 @@ static bool wide_of(const Sim &s, const Level &l)
 //   blocks, the open cells and the rotor cells in the bulk kernel.  Against
 //   groups of open cells, wall cells and rotor cells on side streams: sphere
 //   96x48x48 57 -> 24, 186x92x84 (K17) 86 -> 57, 256x128x128 179 -> 155 (FP16
-//   126 -> 94), two-level rotor duct 427 -> 286.  Levels of up to 32768 cells
-//   keep the groups (48x24x24: 34 against 18): there the open cells have
-//   always been reported as cells of a kernel of their own.
+//   126 -> 94), two-level rotor duct 427 -> 286, and the smallest boxes too:
+//   sphere 48x24x24 34 -> 18.
 // * the levels in order on one stream: three-level sphere 344, with a stream
 //   per level 384.
 // * wall cells on a side stream again on a refined level of more than 200 MiB,
@@ -234,7 +233,7 @@ Sim::Tune tune_of(const Sim &s, const Level &l)
     t.overlap = deep ? 1 : 3;
     t.ordered = true;
     t.rotorInBulk = 1;
-    t.openGroup = l.N > 32768 ? 1 : 0;
+    t.openGroup = 1;
     t.xcdRemap = !l.rotors.empty() || bytes > 512 * MiB ? 2 : 3;
     const bool cap = deep || bytes > 512 * MiB || (!l.openInBulk && bytes > 64 * MiB && bytes <= 256 * MiB);
     t.bulkLds = size >= 4 && cap ? LBM3_BULK_LDS : 0;

@@ -98,7 +98,7 @@ def test_open_cells_in_the_bulk_kernel_equal_the_open_cell_kernel(storage):
     case, dom, tris = _fused_sphere()
     case.trackOpenBoundaries = 1
     runs = []
-    for g, overlap, split in ((0, 1, 0), (1, 1, 0), (1, 0, 0), (1, 1, 2), (1, 0, 2), (1, 1, 3), (1, 3, 0), (0, 3, 0)):
+    for g, overlap, split in ((8, 1, 0), (1, 1, 0), (1, 0, 0), (1, 1, 2), (1, 0, 2), (1, 1, 3), (1, 3, 0), (8, 3, 0), (0, 0, 0)):
         s = lib.Sim(case, storage)
         s.build(dom, tris)
         s.init()
@@ -110,7 +110,8 @@ def test_open_cells_in_the_bulk_kernel_equal_the_open_cell_kernel(storage):
                      s.wall_forces(0)])
         k = s.cell_kinds(0)
         assert k["bulk"] + k["wall"] + k["open_group"] + k["solid"] + k["rotor"] + (k["open"] - k["open_in_bulk"]) == s.info(0).cellCount
-        assert k["open_in_bulk"] == (0 if not g else (k["open"] if split in (0, 3) else k["open_in_bulk"])) and \
+        # (0: nothing set, the open cells in the bulk kernel)
+        assert k["open_in_bulk"] == (0 if g == 8 else (k["open"] if split in (0, 3) else k["open_in_bulk"])) and \
             (split != 2 or 0 < k["open_in_bulk"] < k["open"])
         s.close()
     for other in runs[1:]:

@@ -79,9 +79,8 @@ def test_restart_reproduces_the_pipe_run(tmp_path, storage):
 
 @pytest.mark.parametrize("storage", ["f32", "f16"])
 def test_fresh_restart_with_a_fused_open_level(tmp_path, storage):
-    """Sphere whose open faces touch no wall, so level 0 runs its open cells in
-    the open-cell kernel (the boundary condition of a step completed when the
-    next step loads the cell).  The checkpoint is taken with that condition
+    """Sphere whose open faces touch no wall, so a step's boundary condition is
+    completed when the next step loads the cell, in the bulk kernel.  The checkpoint is taken with that condition
     pending and loaded into a freshly built simulation that has never run;
     the continued runs agree bit for bit."""
     case, dom, tris = cases.sphere(48, 24, 24, diameter=6.0, center=(14.0, 12.0, 12.0), segments=(16, 32))
@@ -90,7 +89,7 @@ def test_fresh_restart_with_a_fused_open_level(tmp_path, storage):
     a.build(dom, tris)
     a.init()
     a.run(17)
-    assert a.cell_kinds(0)["open"] > 0                   # the open cells have their own kernel
+    assert a.cell_kinds(0)["open"] > 0                   # completed at the next load
     path = tmp_path / "sphere.ckpt"
     a.save_checkpoint(path)
     a.run(11)

@@ -95,10 +95,12 @@ def test_short_rows_equal_the_oracle(n):
 
 
 @pytest.mark.parametrize("storage", ["f32", "f16"])
-def test_default_choices_equal_the_side_stream_kernels(storage):
-    """A sphere large enough for the one-launch default (open and wall cells in
-    the bulk kernel's launch) against the kernels of their own: same bits."""
-    case, dom, tris = cases.sphere(70, 34, 32, diameter=9.0, center=(20.0, 17.0, 16.0), segments=(16, 32))
+@pytest.mark.parametrize("dims", [(24, 14, 12), (48, 24, 24), (70, 34, 32)])
+def test_default_choices_equal_the_side_stream_kernels(dims, storage):
+    """The one-launch default (open and wall cells in the bulk kernel's launch),
+    also on the smallest boxes, against the kernels of their own: same bits."""
+    case, dom, tris = cases.sphere(*dims, diameter=dims[1] / 4.0, center=(dims[0] / 4.0, dims[1] / 2.0, dims[2] / 2.0),
+                                   segments=(16, 32))
     out = []
     for chosen in (None, (40960, 2, 1, 8)):
         s = lib.Sim(case, storage)
