@@ -188,7 +188,9 @@ int lbm3_upload_populations(lbm3_sim *s, int level, const void *in, long long by
  * last build, any level).  "cellRow" is the per-step kernels' cell record, 8
  * bytes per cell: {kind, row} with kind >= 0 wall-adjacent entry, -1/-2 bulk,
  * -3 solid, -4 a cell the rotors can reach, <= -8 open cell (the last two
- * updated by kernels of their own).  With out == NULL only
+ * updated by kernels of their own unless the bulk kernel takes them: "rotorBits",
+ * "openBits"); "imageSources" marks the cells whose periodic ghosts the bulk
+ * kernel steps with them (a bit per cell; empty: the ghosts are copied).  With out == NULL only
  * *count is returned. */
 int lbm3_download_array(lbm3_sim *s, int level, const char *name, void *out, long long capacity, long long *count);
 /* The same arrays in device memory, not copied: *ptr points into the

@@ -253,11 +253,18 @@ static int prepare_images(Sim &s, Level &l)
     const long long words = 4 * ((l.N + 255) / 256);
     DBuf<int> flag;
     HIPCHK(flag.alloc(1));
-    HIPCHK(l.ghostSkip.alloc(words));
-    HIPCHK(l.imageSources.alloc(words));
-    HIPCHK(l.imageHead.alloc(l.N));
-    HIPCHK(l.imageInfo.alloc(l.nPeriodic));
-    HIPCHK(l.imageNb.alloc(2LL * l.nPeriodic));
+    // where the tables do not fit beside the level the copy needs none
+    if (l.ghostSkip.alloc(words) != hipSuccess || l.imageSources.alloc(words) != hipSuccess ||
+        l.imageHead.alloc(l.N) != hipSuccess || l.imageInfo.alloc(l.nPeriodic) != hipSuccess ||
+        l.imageNb.alloc(2LL * l.nPeriodic) != hipSuccess) {
+        (void)hipGetLastError();
+        l.ghostSkip.release();
+        l.imageSources.release();
+        l.imageHead.release();
+        l.imageInfo.release();
+        l.imageNb.release();
+        return 0;
+    }
     HIPCHK(hipMemsetAsync(flag.p, 0, sizeof(int), s.stream));
     HIPCHK(hipMemsetAsync(l.imageSources.p, 0, sizeof(uint64_t) * (size_t)words, s.stream));
     HIPCHK(hipMemcpyAsync(l.ghostSkip.p, l.bulkSkip.p, sizeof(uint64_t) * (size_t)words, hipMemcpyDeviceToDevice, s.stream));
@@ -1634,6 +1641,7 @@ int lbm3_download_array(lbm3_sim *h, int level, const char *name, void *out, lon
     ARR("cellRow", l.cellRow, l.N)
     ARR("bulkSkip", l.bulkSkip, (l.N + 63) / 64) ARR("openBits", l.openBits, l.openInBulk ? (l.N + 63) / 64 : 0)
     ARR("rotorBits", l.rotorBits, l.rotorInBulk ? (l.N + 63) / 64 : 0)
+    ARR("imageSources", l.imageSources, l.imagesReady ? (l.N + 63) / 64 : 0)
     ARR("linkLength", l.linkLength, 7LL * l.W) ARR("periodicIndex", l.perIndex, l.nPeriodic)
     ARR("periodicSource", l.perSource, l.nPeriodic) ARR("openIndex", l.openCell, l.nOpen)
     ARR("openSource", l.openSource, l.nOpen) ARR("openMeta", l.openMeta, l.nOpen)

@@ -254,7 +254,7 @@ class Sim:
         n = max(cnt.value, 0)
         if name in ("rayHitScan", "cellRow"):
             dt = np.int64
-        elif name in ("bulkSkip", "openBits"):
+        elif name in ("bulkSkip", "openBits", "imageSources"):
             dt = np.uint64
         elif name.startswith("rotor") and name.endswith("Force"):
             dt = np.float64

@@ -32,12 +32,18 @@ BOXES = {
 }
 
 
+def _sources(s):
+    """Cells whose ghosts the bulk kernel steps; 0: the ghosts are copied."""
+    return int(np.unpackbits(s.array("imageSources", 0).view(np.uint8)).sum())
+
+
 @pytest.mark.parametrize("storage", ["f32", "f64", "f16", "bf16", "f16c"])
 @pytest.mark.parametrize("box", list(BOXES))
 def test_images_equal_the_copy(box, storage):
     a, b = (_make(*BOXES[box](), storage, 3) for _ in range(2))
     for steps in (1, 2, 5, 4):
         a.run(steps)
+        assert _sources(a) == len(np.unique(a.array("periodicSource", 0)))
         b.run_graph(steps)
         got, last = a.populations(0), b.populations(0)
         assert got.tobytes() == last.tobytes(), (steps, np.argwhere(got.view(np.uint8) != last.view(np.uint8))[:4])
@@ -55,6 +61,7 @@ def test_images_with_open_cells_in_the_bulk_kernel():
         s.run(1)
         s.set_tune(0, 2, 1, group)
         s.run(12)
+        assert (_sources(s) > 0) == (group == 1)    # a ghost in a group is another kernel's
         sims.append(s)
     assert sims[0].populations(0).tobytes() == sims[1].populations(0).tobytes()
 
@@ -64,6 +71,7 @@ def test_images_checkpoint_and_graph(tmp_path):
     a, b = (_make(*BOXES["cube 14"](), "f32", 9) for _ in range(2))
     a.run(5)
     b.run(5)
+    assert _sources(a) > 0
     a.save_checkpoint(tmp_path / "c")
     a.run(4)
     a.run_graph(7)
@@ -90,6 +98,7 @@ def test_short_rows_equal_the_oracle(n):
     s.init_fields(0, f.astype(np.float32))
     o.run(21)
     s.run(21)
+    assert _sources(s) > 0
     a, b = o.macros(), s.macros(0)
     assert max(rel_max(1 + b[:, 0], 1 + a[:, 0]), rel_max(b[:, 1:], a[:, 1:])) < 1e-10
 
@@ -112,6 +121,10 @@ def test_default_choices_equal_the_side_stream_kernels(dims, storage):
         assert (s.cell_kinds(0)["open_in_bulk"] > 0) == (chosen is None)
         out.append((s.populations(0).tobytes(), s.wall_forces(0).tobytes()))
     assert out[0] == out[1]
+
+
+def _same(a, b):
+    return a.tobytes() == b.tobytes()
 
 
 class _Kept:
@@ -153,19 +166,20 @@ def test_a_kept_address_sees_and_sets_the_ghosts(box):
     f = _Kept(a)
     first = f.read()
     b.run_graph(4)
-    assert first.tobytes() == b.populations(0).tobytes()
+    assert _same(first, b.populations(0))
     ghosts = a.array("periodicIndex", 0)
+    assert _sources(a) > 0
     for k, step in enumerate((lambda s: s.run(3), lambda s: s.run_graph(5), lambda s: s.run_timed(2, kernel_events=False),
                               lambda s: s.run(1))):
         step(a)
         a.sync()
         now = f.read()
         b.run_graph((3, 5, 2, 1)[k])
-        assert now.tobytes() == b.populations(0).tobytes(), k
+        assert _same(now, b.populations(0)), k
         # the ghosts get other values through the address
         now[:, ghosts[::3]] *= np.float32(1.25)
         f.write(now)
         b.set_populations(0, now)
     a.run(2)
     b.run_graph(2)
-    assert a.populations(0).tobytes() == b.populations(0).tobytes()
+    assert _same(a.populations(0), b.populations(0))
