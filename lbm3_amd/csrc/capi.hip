@@ -201,7 +201,7 @@ static bool wide_of(const Sim &s, const Level &l)
 //   groups of open cells, wall cells and rotor cells on side streams: sphere
 //   96x48x48 57 -> 24, 186x92x84 (K17) 86 -> 57, 256x128x128 179 -> 155 (FP16
 //   126 -> 94), two-level rotor duct 427 -> 286, and the smallest boxes too:
-//   sphere 48x24x24 34 -> 18.
+//   sphere 48x24x24 34 -> 18.  FP64: 48x24x24 48 -> 14, 256x128x128 445 -> 328.
 // * the levels in order on one stream: three-level sphere 344, with a stream
 //   per level 384.
 // * wall cells on a side stream again on a refined level of more than 200 MiB,

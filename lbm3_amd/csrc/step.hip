@@ -893,15 +893,18 @@ __device__ __noinline__ void wall_cell_call(const __attribute__((address_space(4
 // wall path needs about twice the bulk path's registers; the register budget is
 // held to six waves per SIMD (the bulk path fits it, the wall path spills), so
 // the bulk blocks keep their occupancy; at seven the 16-bit bulk path spills too.
-// With the rotor cells inside (103 registers) four waves: more would spill in
-// the rotor path.
-constexpr int walls_waves(bool rotor)
+// With the rotor cells inside (103 registers) four waves: the wall path spills a
+// little (11), at more waves the rotor path would.  FP64 needs 245 registers, two
+// waves: at the FP32 budget its bulk path spilled too (up to 806), sphere 96x48x48
+// 70 us per step against 25, 256x128x128 328 (with the wall cells on a side
+// stream 338 to 362, and the open cells in groups 445).
+template <class S> constexpr int walls_waves(bool rotor)
 {
-    return rotor ? 4 : 6;
+    return sizeof(S) == 8 ? 2 : rotor ? 4 : 6;
 }
 
 template <class S, bool FLIP, int BULK, bool OPEN, bool ROTOR = false>
-__global__ __launch_bounds__(256, walls_waves(ROTOR)) void k_collide_stream_walls(StepArgs<S> a)
+__global__ __launch_bounds__(256, walls_waves<S>(ROTOR)) void k_collide_stream_walls(StepArgs<S> a)
 {
     const int b = blockIdx.x;
     if (b < a.wallBlocks) {
