@@ -140,8 +140,9 @@ int lbm3_synchronize(lbm3_sim *s);
  * other open cells; 3: in the bulk kernel with a block's lanes rotated by 32
  * cells, so that a row's two x-face cells share a wave), and, where a level
  * has rotors, whether the bulk kernel steps the rotor cells too instead of a
- * kernel of their own; times the six fastest again, three rounds in turn, keeps
- * the one with the best round and restores the simulation's state
+ * kernel of their own; times the six fastest and each level's own choices (see
+ * lbm3_get_tune; not in `out`) again, three rounds in turn, keeps
+ * the one with the best round (the levels' own where none is faster) and restores the simulation's state
  * as it was (the populations and every step counter; a
  * pending open-boundary condition stays pending unless the chosen open-cell
  * layout differs, which completes it first).  out[7 r + {LDS bytes,
@@ -149,9 +150,9 @@ int lbm3_synchronize(lbm3_sim *s);
  * bulk kernel, ms per step in the sweep}] for the first `cap` candidates; *nOut the
  * candidates timed. */
 int lbm3_autotune(lbm3_sim *s, int steps, double *out, int cap, int *nOut);
-/* The launch choices in use (until lbm3_set_tune or lbm3_autotune sets them, each
+/* The launch choices in use (until lbm3_set_tune or lbm3_autotune sets others, each
  * level takes its own by its size and cells; lbm3_get_tune then gives level
- * 0's): {bulk LDS bytes, block order, side streams, open
+ * 0's, and setting just those leaves every level its own): {bulk LDS bytes, block order, side streams, open
  * group cells, x-face choice, rotor cells in the bulk kernel}; lbm3_set_tune
  * sets them (LDS 0..65536, block order 0..3, side streams 0..3, group 1, 8 or
  * 16, x-face choice 0..3, rotor cells 0..1; a new layout of the open or rotor

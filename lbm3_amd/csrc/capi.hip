@@ -232,7 +232,8 @@ Sim::Tune tune_of(const Sim &s, const Level &l)
     const bool deep = s.levels > 1 && l.W > 0 && !l.openInBulk && l.rotors.empty() && bytes > 200 * MiB;
     t.overlap = deep ? 1 : 3;
     t.ordered = true;
-    t.rotorInBulk = 1;
+    // the same on every level: a new layout rebuilds all of them (same_open_layout)
+    for (int L = 0; L < s.levels; ++L) t.rotorInBulk |= s.L[L].rotors.empty() ? 0 : 1;
     t.openGroup = 1;
     t.xcdRemap = !l.rotors.empty() || bytes > 512 * MiB ? 2 : 3;
     const bool cap = deep || bytes > 512 * MiB || (!l.openInBulk && bytes > 64 * MiB && bytes <= 256 * MiB);
@@ -1239,19 +1240,47 @@ int lbm3_autotune(lbm3_sim *h, int steps, double *out, int cap, int *nOut)
     for (int r = 0; r < (rotors ? 2 : 1); ++r)
         for (const auto &o : open) groups.push_back({o.first, o.second, r});
     const int ldsChoices[4] = {0, 24576, 40960, 65536};
-    const Sim::Tune start = tune_of(s, s.L[0]);
+    const Sim::Tune start = s.tune;
     const bool startChosen = s.tuneChosen;
-    s.tuneChosen = true;
-    Sim::Tune best = start;
+    // candidate 0: every level's own choices (tune_of), which no single set of
+    // choices gives on several levels: three-level sphere 348 us per step against
+    // 368 for the best single set
+    struct Cand { Sim::Tune t; bool chosen; double ms; };
+    std::vector<Cand> cands;
+    auto layout = [&](bool chosen, const Sim::Tune &t) {
+        s.tuneChosen = chosen;
+        s.tune = t;
+        return tune_of(s, s.L[0]);
+    };
     double bestMs = 1e300;
     int rows = 0;
-    struct Cand { Sim::Tune t; double ms; };
-    std::vector<Cand> cands;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     int rc = 0;
+    // `steps` steps of the choices in use, after one untimed step, ms per step
+    auto timed = [&](double &per) {
+        update_all(s, 0);
+        if (const int e = check_hip(hipEventRecord(e0, s.stream), "event")) return e;
+        for (int k = 0; k < steps; ++k) update_all(s, 0);
+        if (const int e = check_hip(hipEventRecord(e1, s.stream), "event")) return e;
+        if (const int e = check_hip(hipEventSynchronize(e1), "autotune step")) return e;
+        float ms = 0.f;
+        if (const int e = check_hip(hipEventElapsedTime(&ms, e0, e1), "event time")) return e;
+        per = (double)ms / steps;
+        return 0;
+    };
+    {
+        Cand own{start, false, 0.0};
+        const Sim::Tune was = tune_of(s, s.L[0]);
+        if (!same_open_layout(s, was, layout(false, start))) rc = regroup(s);
+        if (!rc) rc = timed(own.ms);
+        cands.push_back(own);
+    }
+    s.tuneChosen = true;
+    s.tune = Sim::Tune{};
     for (const Layout &gs : groups) {
+        if (rc) break;
         const int g = gs.group;
         s.tune.openGroup = g;
         s.tune.openSplit = gs.split;
@@ -1264,20 +1293,14 @@ int lbm3_autotune(lbm3_sim *h, int steps, double *out, int cap, int *nOut)
                     s.tune.bulkLds = lds;
                     s.tune.xcdRemap = remap;
                     s.tune.overlap = overlap;
-                    update_all(s, 0);                     // one untimed step in this configuration
-                    if ((rc = check_hip(hipEventRecord(e0, s.stream), "event"))) break;
-                    for (int k = 0; k < steps; ++k) update_all(s, 0);
-                    if ((rc = check_hip(hipEventRecord(e1, s.stream), "event"))) break;
-                    if ((rc = check_hip(hipEventSynchronize(e1), "autotune step"))) break;
-                    float ms = 0.f;
-                    if ((rc = check_hip(hipEventElapsedTime(&ms, e0, e1), "event time"))) break;
-                    const double per = (double)ms / steps;
+                    double per = 0.0;
+                    if ((rc = timed(per))) break;
                     if (rows < cap) {
                         double *o = out + 7 * (size_t)rows;
                         o[0] = lds; o[1] = remap; o[2] = overlap; o[3] = g; o[4] = gs.split; o[5] = gs.rotor; o[6] = per;
                     }
                     ++rows;
-                    cands.push_back({s.tune, per});
+                    cands.push_back({s.tune, true, per});
                 }
         if (rc) break;
     }
@@ -1285,31 +1308,25 @@ int lbm3_autotune(lbm3_sim *h, int steps, double *out, int cap, int *nOut)
     // and the best of each candidate's rounds decides: a single noisy timing
     // in the sweep (a launch that met another's traffic in the cache, a clock
     // change) does not pick the configuration alone.
-    if (!rc && !cands.empty()) {
-        std::stable_sort(cands.begin(), cands.end(), [](const Cand &a, const Cand &b) { return a.ms < b.ms; });
-        const int K = (int)std::min<size_t>(6, cands.size());
+    // Candidate 0 is always among them and wins ties.
+    int best = 0;
+    if (!rc) {
+        std::stable_sort(cands.begin() + 1, cands.end(), [](const Cand &a, const Cand &b) { return a.ms < b.ms; });
+        const int K = (int)std::min<size_t>(7, cands.size());
         std::vector<double> again(K, 1e300);
         for (int round = 0; round < 3 && !rc; ++round)
             for (int i = 0; i < K && !rc; ++i) {
-                const bool relayout = !same_open_layout(s, s.tune, cands[i].t);
-                s.tune = cands[i].t;
-                if (relayout && (rc = regroup(s))) break;
-                update_all(s, 0);
-                if ((rc = check_hip(hipEventRecord(e0, s.stream), "event"))) break;
-                for (int k = 0; k < steps; ++k) update_all(s, 0);
-                if ((rc = check_hip(hipEventRecord(e1, s.stream), "event"))) break;
-                if ((rc = check_hip(hipEventSynchronize(e1), "autotune step"))) break;
-                float ms = 0.f;
-                if ((rc = check_hip(hipEventElapsedTime(&ms, e0, e1), "event time"))) break;
-                again[i] = std::min(again[i], (double)ms / steps);
+                const Sim::Tune was = tune_of(s, s.L[0]);
+                if (!same_open_layout(s, was, layout(cands[i].chosen, cands[i].t)) && (rc = regroup(s))) break;
+                double per = 0.0;
+                if (!(rc = timed(per))) again[i] = std::min(again[i], per);
             }
         for (int i = 0; i < K; ++i)
-            if (again[i] < bestMs) { bestMs = again[i]; best = cands[i].t; }
+            if (again[i] < bestMs) { bestMs = again[i]; best = i; }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    s.tune = start;
-    s.tuneChosen = startChosen;
+    const Sim::Tune was = layout(startChosen, start);
     const int rg = regroup(s);
     const int rs = restore_snapshot(s, z);
     if (rc) return rc;
@@ -1318,20 +1335,30 @@ int lbm3_autotune(lbm3_sim *h, int steps, double *out, int cap, int *nOut)
     if (nOut) *nOut = rows;
     // another open-cell layout: the pending condition is completed in the old
     // one first (regroup), which rounds it to the storage type once
-    const bool relayout = !same_open_layout(s, start, best);
-    s.tune = best;
-    s.tuneChosen = true;
-    return relayout ? regroup(s) : 0;
+    return same_open_layout(s, was, layout(cands[best].chosen, cands[best].t)) ? 0 : regroup(s);
+}
+
+// level 0's choices, as lbm3_get_tune reports them: by its cells' records, which
+// the first step makes
+static int reported_tune(Sim &s, int (&t6)[6])
+{
+    Level &l = s.L[0];
+    if (!s.tuneChosen && l.built && !l.openFusionChecked)
+        if (const int rc = prepare_open_fusion(s, 0)) return rc;
+    const Sim::Tune t = tune_of(s, l);
+    t6[0] = t.bulkLds; t6[1] = t.xcdRemap; t6[2] = t.overlap;
+    t6[3] = t.openGroup ? t.openGroup : open_group_cells((int)storage_bytes(s.storage));
+    t6[4] = t.openSplit;
+    t6[5] = t.rotorInBulk;
+    return 0;
 }
 
 int lbm3_get_tune(lbm3_sim *h, int *out6)
 {
     if (!h || !out6) return set_error(LBM3_E_ARG, "null argument");
-    const Sim::Tune t = tune_of(h->s, h->s.L[0]);
-    out6[0] = t.bulkLds; out6[1] = t.xcdRemap; out6[2] = t.overlap;
-    out6[3] = t.openGroup ? t.openGroup : open_group_cells((int)storage_bytes(h->s.storage));
-    out6[4] = t.openSplit;
-    out6[5] = t.rotorInBulk;
+    int t[6];
+    if (const int rc = reported_tune(h->s, t)) return rc;
+    memcpy(out6, t, sizeof t);
     return 0;
 }
 
@@ -1345,6 +1372,12 @@ int lbm3_set_tune(lbm3_sim *h, const int *in6)
                                      "kernel), 8 or 16 cells, x-face choice 0..3, rotor cells 0..1");
     Sim &s = h->s;
     if (s.timing) return set_error(LBM3_E_STATE, "launch choices changed during a timed run");
+    if (!s.tuneChosen) {
+        // what lbm3_get_tune reports leaves every level its own choices
+        int now[6];
+        if (const int rc = reported_tune(s, now)) return rc;
+        if (memcmp(now, in6, sizeof now) == 0) return 0;
+    }
     const Sim::Tune was = tune_of(s, s.L[0]);
     s.tuneChosen = true;
     s.tune = Sim::Tune{};
