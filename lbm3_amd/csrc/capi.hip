@@ -235,6 +235,7 @@ Sim::Tune tune_of(const Sim &s, const Level &l)
     // the same on every level: a new layout rebuilds all of them (same_open_layout)
     for (int L = 0; L < s.levels; ++L) t.rotorInBulk |= s.L[L].rotors.empty() ? 0 : 1;
     t.openGroup = 1;
+    t.openSplit = s.ownSplit;
     t.xcdRemap = !l.rotors.empty() || bytes > 512 * MiB ? 2 : 3;
     const bool cap = deep || bytes > 512 * MiB || (!l.openInBulk && bytes > 64 * MiB && bytes <= 256 * MiB);
     t.bulkLds = size >= 4 && cap ? LBM3_BULK_LDS : 0;
@@ -2113,9 +2114,7 @@ int lbm3_load_checkpoint(lbm3_sim *h, const char *path)
         Level &l = s.L[L];
         if (settled[(size_t)L] || !l.fusedOpen || split[(size_t)L] == (l.nSepEntries > 0)) continue;
         if (const int rc = settle_open(s, L)) { fclose(fp); return rc; }
-        s.tune = tune_of(s, l);
-        s.tuneChosen = true;
-        s.tune.openSplit = split[(size_t)L] ? 1 : 0;
+        (s.tuneChosen ? s.tune.openSplit : s.ownSplit) = split[(size_t)L] ? 1 : 0;
         l.openFusionChecked = false;
         if (const int rc = prepare_open_fusion(s, L)) { fclose(fp); return rc; }
     }

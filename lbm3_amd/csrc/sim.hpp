@@ -176,6 +176,7 @@ struct Sim {
         bool ordered = false;         // overlap 3 with the levels in order on one stream (tune_of)
     } tune;
     bool tuneChosen = false;         // the caller or the autotuner set `tune`; else every level takes tune_of's rule
+    int ownSplit = 0;                // Tune::openSplit of that rule: a loaded checkpoint's pending condition decides it
     // graph capture: each level step takes the next slot of this device table
     // for the values that change between replays; a dry run only collects them
     StepParam *captureTable = nullptr;

@@ -1,5 +1,5 @@
 """The levels' own launch choices (nothing set) against lbm3_get_tune,
-lbm3_set_tune and lbm3_autotune."""
+lbm3_set_tune, lbm3_autotune and a loaded checkpoint."""
 import numpy as np
 import pytest
 
@@ -56,4 +56,26 @@ def test_set_and_autotuned_choices_are_not_slower_on_three_levels():
     print("three levels, ms per 20 steps: own %.3f, set as reported %.3f, autotuned %.3f" % (a, b, c))
     assert b < 1.04 * a and c < 1.04 * a
     for s in (own, same, tuned):
+        s.close()
+
+
+def test_a_loaded_x_face_split_changes_no_other_choice(tmp_path):
+    """A checkpoint with a condition pending for the split layout: the loading
+    simulation adopts the split, keeps its other choices and continues bit for bit."""
+    make = lambda: cases.sphere(48, 24, 24, diameter=6.0, center=(14.0, 12.0, 12.0), segments=(16, 32))
+    a, b = _sim(make), _sim(make)
+    a.set_tune(40960, 0, 1, 8, 1)
+    a.run(9)
+    a.save_checkpoint(tmp_path / "c")
+    a.run(6)
+    own = b.tune()
+    b.load_checkpoint(tmp_path / "c")
+    assert b.tune() == dict(own, open_split=1)
+    b.run(6)
+    assert np.array_equal(a.macros(0), b.macros(0))
+    # still the levels' own: another layout, and back by setting what is reported
+    t = b.tune()
+    b.set_tune(*(t[k] for k in lib.Sim.TUNE))
+    assert b.tune() == t
+    for s in (a, b):
         s.close()
