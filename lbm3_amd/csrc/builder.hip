@@ -49,14 +49,18 @@ template <class F> void for_n(long long n, hipStream_t s, F f)
 // item walks as one chain of dependent loads
 template <class F> __global__ __launch_bounds__(256) void k_wave_for(long long n, F f)
 {
-    const long long i = (long long)blockIdx.x * 4 + threadIdx.x / 64;
-    if (i < n) f(i, (int)(threadIdx.x % 64));
+    for (long long i = (long long)blockIdx.x * 4 + threadIdx.x / 64; i < n; i += (long long)gridDim.x * 4) {
+        f(i, (int)(threadIdx.x % 64));
+        __builtin_amdgcn_wave_barrier();   // an item's LDS is read before the next item clears it
+    }
 }
 
+// at most 4096 blocks (16 per CU), whose waves take several items each beyond: a launch holds fewer than
+// 2^32 threads, which one wave per item passes at 67M triangles
 template <class F> void for_waves(long long n, hipStream_t s, F f)
 {
     if (n <= 0) return;
-    hipLaunchKernelGGL((k_wave_for<F>), dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, n, f);
+    hipLaunchKernelGGL((k_wave_for<F>), dim3((unsigned)std::min<long long>(4096, (n + 3) / 4)), dim3(256), 0, s, n, f);
 }
 
 // the lowest and highest of three values per item over all items: out[2 a] and

@@ -1,7 +1,8 @@
 """Builder kernels that give each triangle or wall-adjacent cell a wave, on the
 GPU against the oracle, bit for bit: bins of fewer and of many more triangles
 than a wave has lanes, triangles in one bin and in hundreds, one and two
-bodies, one and two levels."""
+bodies, one and two levels, more triangles and wall-adjacent cells than the
+launch has waves (16384)."""
 import numpy as np
 import pytest
 
@@ -33,6 +34,8 @@ CASES = {
     "120x240, most of them in each bin's reach": lambda: _sphere((120, 240), 16),
     "60x120 on two levels": lambda: _sphere((60, 120), levels=2),
     "two bodies": _two_bodies,
+    "more items than waves": lambda: (lambda c: (c[0], c[1], [geometry.uv_sphere(33.0, (40.2, 40.1, 39.7), 100, 200)]))(
+        _sphere((4, 8), 80)),
 }
 
 
@@ -47,4 +50,4 @@ def test_walls_and_links_equal_the_oracle(name):
             assert np.array_equal(s.array(a, level), o.array(a, level)), (level, a)
         b, c = s.info(level).Bounds, o.info(level).Bounds
         assert [getattr(b, k) for k, _ in b._fields_] == [getattr(c, k) for k, _ in c._fields_]
-    assert s.array("wallIndex", case.gridLevelCount - 1).size > 0
+    assert s.array("wallIndex", case.gridLevelCount - 1).size > (16384 if name == "more items than waves" else 0)
