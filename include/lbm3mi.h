@@ -160,7 +160,9 @@ int lbm3_autotune(lbm3_sim *s, int steps, double *out, int cap, int *nOut);
  * pending open-boundary condition first).  Every choice gives the
  * same results bit for bit, except with 16-bit storage: that completion, and
  * every step's separate pass for the x faces, store the completed populations
- * rounded to the storage type. */
+ * rounded to the storage type; and except the rotor choice, which compiles the
+ * collision of the waves holding rotor cells twice: there up to the rounding of
+ * its multiply-adds. */
 int lbm3_get_tune(lbm3_sim *s, int *out6);
 int lbm3_set_tune(lbm3_sim *s, const int *in6);
 

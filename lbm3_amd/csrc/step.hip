@@ -450,7 +450,11 @@ __device__ __forceinline__ short half_of(const unsigned (&bits)[14], int q) { re
 // instead of 21.1 (FP32, fastest launch choices of each), FP16 106^3 37.0
 // instead of 43.2, the 256x64x64 duct in BF16 34.5 instead of 40.3; the rows of
 // a wave in one scalar load (row_in_wave) take them to 14.8, 35.1 and 32.7.
-template <class S, bool FLIP, int BULK, class Off, bool OPEN = false, bool ROTOR = false, bool ROT = false, bool IMG = false>
+// DEV: 16-bit storage collides the stored deviations (deviation_cell).  Not on a
+// level with rotors, whose cells collide their populations whichever kernel
+// steps them (lbm3_set_tune's rotor choice), nor above 4 GiB.
+template <class S, bool FLIP, int BULK, class Off, bool OPEN = false, bool ROTOR = false, bool ROT = false, bool IMG = false,
+          bool DEV = true>
 __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell, const StepNow &now)
 {
     using T = typename StoreTraits<S>::compute;
@@ -483,7 +487,7 @@ __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell, const 
     if constexpr (sizeof(Off) == 4 && (sizeof(S) >= 4 || LBM3_BUF16 > 0)) {
         // raw buffer accesses: the plane offset is a scalar operand
         const __amdgpu_buffer_rsrc_t r = pop_rsrc(a.f, 27LL * padded_cells(a.fast.N) * (long long)sizeof(S));
-        if constexpr (sizeof(S) == 2 && !ROTOR) {
+        if constexpr (sizeof(S) == 2 && !ROTOR && DEV) {
             unsigned bits[14];
             bool open = false;
             if constexpr (OPEN) open = now.pending && mask_bit<ROT>(a.fast.openBits, cell);
@@ -563,14 +567,15 @@ __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell, const 
 // row -- both x-face cells -- share one wave, which then runs the open
 // condition once for the two instead of two waves once each; every access of
 // that wave still fills whole 128-byte lines
-template <class S, bool FLIP, int BULK, bool WIDE, bool OPEN = false, bool ROTOR = false, bool ROT = false, bool IMG = false>
+template <class S, bool FLIP, int BULK, bool WIDE, bool OPEN = false, bool ROTOR = false, bool ROT = false, bool IMG = false,
+          bool DEV = true>
 __global__ __launch_bounds__(256) void k_collide_stream(StepArgs<S> a)
 {
     const int lane = ROT ? int((threadIdx.x + 32) & 255) : int(threadIdx.x);
     const int cell = xcd_block(blockIdx.x, gridDim.x, a.xcdRemap, FLIP) * 256 + lane;
     if (cell >= a.fast.N) return;
     if (WIDE) bulk_cell<S, FLIP, BULK, uint64_t>(a, cell, step_now(a));
-    else bulk_cell<S, FLIP, BULK, uint32_t, OPEN, ROTOR, ROT, IMG>(a, cell, step_now(a));
+    else bulk_cell<S, FLIP, BULK, uint32_t, OPEN, ROTOR, ROT, IMG, DEV>(a, cell, step_now(a));
 }
 
 // Open-boundary cells (never wall-adjacent when this kernel is used): load,
@@ -581,7 +586,7 @@ __global__ __launch_bounds__(256) void k_collide_stream(StepArgs<S> a)
 // fluid cell of the group (record -5 or <= -8); a wave covers 64 / G groups,
 // sorted so that they share one boundary condition and normal, so the
 // boundary-condition code runs once per wave for all its open lanes.
-template <class S, bool FLIP, int BULK, int G>
+template <class S, bool FLIP, int BULK, int G, bool DEV = true>
 __global__ __launch_bounds__(256) void k_open_groups(StepArgs<S> a)
 {
     using T = typename StoreTraits<S>::compute;
@@ -599,7 +604,7 @@ __global__ __launch_bounds__(256) void k_open_groups(StepArgs<S> a)
     for (int k = 0; k < 8; ++k)
         off[k] = ((uint32_t(nb[k]) / LBM3_TILE) * uint32_t(27 * LBM3_TILE) + uint32_t(nb[k]) % LBM3_TILE) * uint32_t(sizeof(S));
     const __amdgpu_buffer_rsrc_t r = pop_rsrc(a.f, 27LL * padded_cells(a.fast.N) * (long long)sizeof(S));
-    if constexpr (sizeof(S) == 2) {
+    if constexpr (sizeof(S) == 2 && DEV) {
         unsigned bits[14];
         deviation_cell<S, FLIP, BULK, true>(a, a.param ? a.param->iter : a.open.iter, cell,
                                             code <= -8 && (a.param ? a.param->pending : a.open.pending), r, off, bits);
@@ -903,7 +908,7 @@ template <class S> constexpr int walls_waves(bool rotor)
     return sizeof(S) == 8 ? 2 : rotor ? 4 : 6;
 }
 
-template <class S, bool FLIP, int BULK, bool OPEN, bool ROTOR = false>
+template <class S, bool FLIP, int BULK, bool OPEN, bool ROTOR = false, bool DEV = true>
 __global__ __launch_bounds__(256, walls_waves<S>(ROTOR)) void k_collide_stream_walls(StepArgs<S> a)
 {
     const int b = blockIdx.x;
@@ -922,7 +927,7 @@ __global__ __launch_bounds__(256, walls_waves<S>(ROTOR)) void k_collide_stream_w
     }
     const int cell = xcd_block(b - a.wallBlocks, gridDim.x - a.wallBlocks, a.xcdRemap, FLIP) * 256 + threadIdx.x;
     if (cell >= a.fast.N) return;
-    bulk_cell<S, FLIP, BULK, uint32_t, OPEN, ROTOR>(a, cell, step_now(a));
+    bulk_cell<S, FLIP, BULK, uint32_t, OPEN, ROTOR, false, false, DEV>(a, cell, step_now(a));
 }
 
 // derive the hot-loop topology records from the compressed IJK/NBR arrays;
@@ -1455,10 +1460,9 @@ void launch_collide_wall(const StepArgs<S> &a, bool flip, hipStream_t s)
 }
 
 
-template <class S>
-void launch_collide_stream(const StepArgs<S> &a, bool flip, hipStream_t s)
+template <class S, bool DEV>
+static void launch_bulk(const StepArgs<S> &a, bool flip, hipStream_t s)
 {
-    if (a.fast.N <= 0) return;
     const dim3 g(blocks_for(a.fast.N)), b(256);
     const unsigned lds = (unsigned)a.bulkLds;
     const bool k17 = relax_of<typename StoreTraits<S>::compute>(a.bulk).k17 != 0;
@@ -1466,14 +1470,15 @@ void launch_collide_stream(const StepArgs<S> &a, bool flip, hipStream_t s)
     if (a.wallBlocks > 0) {
         // the caller combines only levels without rotated lanes or 64-bit offsets
         const dim3 gw(blocks_for(a.fast.N) + (unsigned)a.wallBlocks);
-#define LBM3_BULK_WALLS(F, K, O) hipLaunchKernelGGL((k_collide_stream_walls<S, F, K, O>), gw, b, lds, s, a)
+#define LBM3_BULK_WALLS(F, K, O) hipLaunchKernelGGL((k_collide_stream_walls<S, F, K, O, false, DEV>), gw, b, lds, s, a)
 #define LBM3_BULK_WALLS_ROTOR(F, K) hipLaunchKernelGGL((k_collide_stream_walls<S, F, K, false, true>), gw, b, lds, s, a)
         const bool o = a.fast.openBits != nullptr;
-        if (a.fast.rotorBits) {
-            if (flip) { if (k17) LBM3_BULK_WALLS_ROTOR(true, 1); else LBM3_BULK_WALLS_ROTOR(true, 2); }
-            else { if (k17) LBM3_BULK_WALLS_ROTOR(false, 1); else LBM3_BULK_WALLS_ROTOR(false, 2); }
-            return;
-        }
+        if constexpr (DEV)
+            if (a.fast.rotorBits) {
+                if (flip) { if (k17) LBM3_BULK_WALLS_ROTOR(true, 1); else LBM3_BULK_WALLS_ROTOR(true, 2); }
+                else { if (k17) LBM3_BULK_WALLS_ROTOR(false, 1); else LBM3_BULK_WALLS_ROTOR(false, 2); }
+                return;
+            }
 #undef LBM3_BULK_WALLS_ROTOR
         if (flip) { if (k17) { if (o) LBM3_BULK_WALLS(true, 1, true); else LBM3_BULK_WALLS(true, 1, false); }
                     else { if (o) LBM3_BULK_WALLS(true, 2, true); else LBM3_BULK_WALLS(true, 2, false); } }
@@ -1482,30 +1487,38 @@ void launch_collide_stream(const StepArgs<S> &a, bool flip, hipStream_t s)
 #undef LBM3_BULK_WALLS
         return;
     }
-#define LBM3_BULK_LAUNCH(F, K, W) hipLaunchKernelGGL((k_collide_stream<S, F, K, W>), g, b, lds, s, a)
-#define LBM3_BULK_OPEN(F, K) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, true>), g, b, lds, s, a)
-#define LBM3_BULK_OPEN_ROT(F, K) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, true, false, true>), g, b, lds, s, a)
+#define LBM3_BULK_LAUNCH(F, K, W) hipLaunchKernelGGL((k_collide_stream<S, F, K, W, false, false, false, false, DEV>), g, b, lds, s, a)
+#define LBM3_BULK_OPEN(F, K) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, true, false, false, false, DEV>), g, b, lds, s, a)
+#define LBM3_BULK_OPEN_ROT(F, K) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, true, false, true, false, DEV>), g, b, lds, s, a)
 #define LBM3_BULK_IMG(F, K, O) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, O, false, false, true>), g, b, lds, s, a)
 #define LBM3_BULK_ROTOR(F, K) hipLaunchKernelGGL((k_collide_stream<S, F, K, false, false, true>), g, b, lds, s, a)
-    if (a.fast.images.sources) {
-        // the level is neither wide nor has rotor cells, rotated lanes or wall-adjacent cells (prepare_images)
-        const bool o = a.fast.openBits != nullptr;
-        if (flip) { if (k17) { if (o) LBM3_BULK_IMG(true, 1, true); else LBM3_BULK_IMG(true, 1, false); }
-                    else { if (o) LBM3_BULK_IMG(true, 2, true); else LBM3_BULK_IMG(true, 2, false); } }
-        else { if (k17) { if (o) LBM3_BULK_IMG(false, 1, true); else LBM3_BULK_IMG(false, 1, false); }
-               else { if (o) LBM3_BULK_IMG(false, 2, true); else LBM3_BULK_IMG(false, 2, false); } }
-    } else if (a.fast.rotorBits && !wide) {
-        if (flip) { if (k17) LBM3_BULK_ROTOR(true, 1); else LBM3_BULK_ROTOR(true, 2); }
-        else { if (k17) LBM3_BULK_ROTOR(false, 1); else LBM3_BULK_ROTOR(false, 2); }
-    } else if (a.fast.openBits && !wide && a.laneRot) {
+    if constexpr (DEV) {
+        if (a.fast.images.sources) {
+            // the level is neither wide nor has rotor cells, rotated lanes or wall-adjacent cells (prepare_images)
+            const bool o = a.fast.openBits != nullptr;
+            if (flip) { if (k17) { if (o) LBM3_BULK_IMG(true, 1, true); else LBM3_BULK_IMG(true, 1, false); }
+                        else { if (o) LBM3_BULK_IMG(true, 2, true); else LBM3_BULK_IMG(true, 2, false); } }
+            else { if (k17) { if (o) LBM3_BULK_IMG(false, 1, true); else LBM3_BULK_IMG(false, 1, false); }
+                   else { if (o) LBM3_BULK_IMG(false, 2, true); else LBM3_BULK_IMG(false, 2, false); } }
+            return;
+        }
+        if (a.fast.rotorBits && !wide) {
+            if (flip) { if (k17) LBM3_BULK_ROTOR(true, 1); else LBM3_BULK_ROTOR(true, 2); }
+            else { if (k17) LBM3_BULK_ROTOR(false, 1); else LBM3_BULK_ROTOR(false, 2); }
+            return;
+        }
+        if (wide) {
+            if (flip) { if (k17) LBM3_BULK_LAUNCH(true, 1, true); else LBM3_BULK_LAUNCH(true, 2, true); }
+            else { if (k17) LBM3_BULK_LAUNCH(false, 1, true); else LBM3_BULK_LAUNCH(false, 2, true); }
+            return;
+        }
+    }
+    if (a.fast.openBits && a.laneRot) {
         if (flip) { if (k17) LBM3_BULK_OPEN_ROT(true, 1); else LBM3_BULK_OPEN_ROT(true, 2); }
         else { if (k17) LBM3_BULK_OPEN_ROT(false, 1); else LBM3_BULK_OPEN_ROT(false, 2); }
-    } else if (a.fast.openBits && !wide) {
+    } else if (a.fast.openBits) {
         if (flip) { if (k17) LBM3_BULK_OPEN(true, 1); else LBM3_BULK_OPEN(true, 2); }
         else { if (k17) LBM3_BULK_OPEN(false, 1); else LBM3_BULK_OPEN(false, 2); }
-    } else if (wide) {
-        if (flip) { if (k17) LBM3_BULK_LAUNCH(true, 1, true); else LBM3_BULK_LAUNCH(true, 2, true); }
-        else { if (k17) LBM3_BULK_LAUNCH(false, 1, true); else LBM3_BULK_LAUNCH(false, 2, true); }
     } else {
         if (flip) { if (k17) LBM3_BULK_LAUNCH(true, 1, false); else LBM3_BULK_LAUNCH(true, 2, false); }
         else { if (k17) LBM3_BULK_LAUNCH(false, 1, false); else LBM3_BULK_LAUNCH(false, 2, false); }
@@ -1517,6 +1530,24 @@ void launch_collide_stream(const StepArgs<S> &a, bool flip, hipStream_t s)
 #undef LBM3_BULK_IMG
 }
 
+// whether a level of 16-bit storage collides populations in every kernel: see bulk_cell
+template <class S> static bool on_populations(const StepArgs<S> &a)
+{
+    return sizeof(S) == 2 && a.nRotors > 0 && !a.fast.rotorBits && !wide_level<S>(a.fast.N);
+}
+
+template <class S>
+void launch_collide_stream(const StepArgs<S> &a, bool flip, hipStream_t s)
+{
+    if (a.fast.N <= 0) return;
+    if constexpr (sizeof(S) == 2)
+        if (on_populations(a)) {
+            launch_bulk<S, false>(a, flip, s);
+            return;
+        }
+    launch_bulk<S, true>(a, flip, s);
+}
+
 template <class S>
 void launch_rotor_cells(const StepArgs<S> &a, bool flip, hipStream_t s)
 {
@@ -1525,13 +1556,15 @@ void launch_rotor_cells(const StepArgs<S> &a, bool flip, hipStream_t s)
     else hipLaunchKernelGGL((k_rotor_cells<S, false>), dim3(blocks_for(a.rotorCellCount)), dim3(256), 0, s, a);
 }
 
-template <class S, int G>
-void launch_open_groups(const StepArgs<S> &a, bool flip, hipStream_t s)
+template <class S, int G, bool DEV>
+static void launch_open_groups(const StepArgs<S> &a, bool flip, hipStream_t s)
 {
     const dim3 g((unsigned)((a.open.count + 256 / G - 1) / (256 / G))), b(256);
     const bool k17 = relax_of<typename StoreTraits<S>::compute>(a.bulk).k17 != 0;
-    if (flip) { if (k17) hipLaunchKernelGGL((k_open_groups<S, true, 1, G>), g, b, 0, s, a); else hipLaunchKernelGGL((k_open_groups<S, true, 2, G>), g, b, 0, s, a); }
-    else { if (k17) hipLaunchKernelGGL((k_open_groups<S, false, 1, G>), g, b, 0, s, a); else hipLaunchKernelGGL((k_open_groups<S, false, 2, G>), g, b, 0, s, a); }
+#define LBM3_GROUPS(F, K) hipLaunchKernelGGL((k_open_groups<S, F, K, G, DEV>), g, b, 0, s, a)
+    if (flip) { if (k17) LBM3_GROUPS(true, 1); else LBM3_GROUPS(true, 2); }
+    else { if (k17) LBM3_GROUPS(false, 1); else LBM3_GROUPS(false, 2); }
+#undef LBM3_GROUPS
 }
 
 // the group widths the open-cell groups may be built with (Sim::Tune::openGroup)
@@ -1539,8 +1572,14 @@ template <class S>
 void launch_open_cells(const StepArgs<S> &a, bool flip, hipStream_t s)
 {
     if (a.open.count <= 0) return;
-    if (a.open.groupCells == 16) launch_open_groups<S, 16>(a, flip, s);
-    else launch_open_groups<S, 8>(a, flip, s);
+    if constexpr (sizeof(S) == 2)
+        if (a.nRotors > 0) {
+            if (a.open.groupCells == 16) launch_open_groups<S, 16, false>(a, flip, s);
+            else launch_open_groups<S, 8, false>(a, flip, s);
+            return;
+        }
+    if (a.open.groupCells == 16) launch_open_groups<S, 16, true>(a, flip, s);
+    else launch_open_groups<S, 8, true>(a, flip, s);
 }
 
 // velocity profile factor of each open-list entry: its rule's radial profile

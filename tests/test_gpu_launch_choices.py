@@ -79,3 +79,37 @@ def test_a_loaded_x_face_split_changes_no_other_choice(tmp_path):
     assert b.tune() == t
     for s in (a, b):
         s.close()
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16", "f16c"])
+@pytest.mark.parametrize("layout", [(40960, 2, 1, 8, 0), (0, 3, 3, 1, 0), (0, 3, 1, 1, 3), (0, 2, 3, 16, 0)])
+def test_rotor_choice_leaves_the_other_cells_of_16_bit_levels(layout, storage):
+    """Whether the bulk kernel steps the rotor cells or a kernel of their own does,
+    the cells that share no wave with them collide with the same arithmetic:
+    after one step the same bits."""
+    case, dom, statics, rotor, info = cases.rotor_duct(192, 24, 24, seed=1, levels=1, n_theta=128, n_axial=8)
+    out = []
+    for in_bulk in (0, 1):
+        s = lib.Sim(case, storage)
+        s.build(dom, statics)
+        s.build_rotors([rotor])
+        s.set_rotor(0, 0, info["omega"], info["axis"], info["origin"])
+        s.init_fields(0, ((np.random.RandomState(5).rand(s.info(0).cellCount, 4) - 0.5) *
+                          np.array([0.004, 0.04, 0.04, 0.04])).astype(np.float32))
+        s.set_tune(*layout, in_bulk)
+        s.run(1)
+        kind = (s.array("cellRow", 0) & 0xFFFFFFFF).astype(np.uint32).view(np.int32)
+        out.append(s.populations(0).view(np.uint16))
+        shifter, row_i = s.array("shifter", 0), s.array("rowI", 0)
+        s.close()
+    a, b = out
+    # cells (rows lie along x) more than a wave from the rotor's, and its slots
+    head = np.maximum.accumulate(np.where(shifter >= 0, np.arange(kind.size), 0))
+    x = row_i[shifter[head]] + np.arange(kind.size) - head
+    rotor_x = x[kind == -4]
+    far = (x > rotor_x.max() + 66) | (x < rotor_x.min() - 66)
+    wave = np.arange(kind.size) // 64
+    far &= ~np.isin(wave, np.unique(wave[kind == -4]))
+    far &= (kind == -1) | (kind == -2) | (kind <= -5)
+    assert far.sum() > 1000
+    assert np.array_equal(a[:, far], b[:, far])
