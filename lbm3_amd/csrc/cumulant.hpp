@@ -349,7 +349,7 @@ template <int MODE>
 __device__ __forceinline__ void collide_deviations(const float (&s)[9], const float (&d)[9], const float (&k)[9],
                                                    const float (&U)[3], const Relax<float> &R, float (&h)[27])
 {
-    constexpr float n = 1.f / 216.f, third = 1.f / 3.f, ninth = 1.f / 9.f, r27 = 1.f / 27.f;
+    constexpr float n = 1.f / 216.f, third = 1.f / 3.f, ninth = 1.f / 9.f;
     auto quad = [](float m, float z, float p) { return __builtin_fmaf(4.f, z, p + m); };
     // ---- density and momentum of h, velocity ----
     const float X0 = quad(k[0], k[1], k[2]), X1 = quad(k[3], k[4], k[5]), X2 = quad(k[6], k[7], k[8]);
@@ -431,7 +431,6 @@ __device__ __forceinline__ void collide_deviations(const float (&s)[9], const fl
     const float pxy = exy + ninth, pxz = exz + ninth, pyz = eyz + ninth;
     M.m122 = __builtin_fmaf(vx, pyz, M.m122); M.m212 = __builtin_fmaf(vy, pxz, M.m212); M.m221 = __builtin_fmaf(vz, pxy, M.m221);
     M.m222 -= __builtin_fmaf(vx2, pyz, third * eyz);
-    (void)r27;
     // ---- back transform: x, y, z; the outer two outputs doubled ----
     auto back = [](float k0, float k1, float k2, float u, float t, float u2, float &m, float &z, float &p) {
         const float S = __builtin_fmaf(k0, u2, __builtin_fmaf(t, k1, k2)), D = __builtin_fmaf(k0, u, k1);

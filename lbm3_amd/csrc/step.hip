@@ -324,14 +324,10 @@ __device__ __forceinline__ void bulk_collide(const StepArgs<S> &a, int cell, int
 // the level on the host (1: K17, 2: K15).  Topology record >= 0: wall-adjacent,
 // -3: solid, -4: a cell the rotors can reach, -5: a fluid cell in a group of
 // open cells, <= -8: open cell (each with its own kernel).
-// 16-bit storage in the bulk kernel: 0 global loads and stores, 1 raw buffer
-// loads and stores, 2 buffer loads and global stores.  Measured on the
-// 256x128x128 sphere (FP16 bulk kernel with the open cells inside, after the
-// stores' plain conversion): 103.2 us, 98.0 us, 99.8 us (with the fused
-// conversion the order was reversed: 93.4, 97.6, 94.4 us, open cells in groups).
-#ifndef LBM3_BUF16
-#define LBM3_BUF16 1
-#endif
+// Raw buffer loads and stores below 4 GiB.  16-bit storage on the 256x128x128
+// sphere (FP16 bulk kernel with the open cells inside, after the stores' plain
+// conversion): 98.0 us, with global loads and stores 103.2, with buffer loads
+// and global stores 99.8.
 
 // OPEN: the level's open cells are in the bulk kernel too (FastTopo::openBits):
 // such a cell first completes the populations the previous step left unknown,
@@ -484,7 +480,7 @@ __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell, const 
 #pragma unroll
     for (int k = 0; k < 8; ++k) off[k] = slot_offset<S, Off>(nb[k]);
     T f[27];
-    if constexpr (sizeof(Off) == 4 && (sizeof(S) >= 4 || LBM3_BUF16 > 0)) {
+    if constexpr (sizeof(Off) == 4) {
         // raw buffer accesses: the plane offset is a scalar operand
         const __amdgpu_buffer_rsrc_t r = pop_rsrc(a.f, 27LL * padded_cells(a.fast.N) * (long long)sizeof(S));
         if constexpr (sizeof(S) == 2 && !ROTOR && DEV) {
@@ -523,30 +519,24 @@ __device__ __forceinline__ void bulk_cell(const StepArgs<S> &a, int cell, const 
         }
         open_in_bulk<S, OPEN, ROT>(a, now, cell, f);
         bulk_collide<S, BULK, ROTOR>(a, cell, row, f);
-        if constexpr (sizeof(S) >= 4 || LBM3_BUF16 == 1) {
 #pragma unroll
-            for (int q = 0; q < 27; ++q)
-                StoreTraits<S>::bstore(r, off[post_nb(q)], post_plane(q, FLIP) * LBM3_TILE * int(sizeof(S)), f[q], q, a.cd);
-            if constexpr (IMG) {
-                while (img >= 0) {
-                    const int gn[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+        for (int q = 0; q < 27; ++q)
+            StoreTraits<S>::bstore(r, off[post_nb(q)], post_plane(q, FLIP) * LBM3_TILE * int(sizeof(S)), f[q], q, a.cd);
+        if constexpr (IMG) {
+            while (img >= 0) {
+                const int gn[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
-                    for (int q = 1; q < 27; ++q)
-                        if ((gi.x >> q) & 1)
-                            StoreTraits<S>::bstore(r, slot_offset<S, Off>(gn[post_nb(q)]),
-                                                   post_plane(q, FLIP) * LBM3_TILE * int(sizeof(S)), f[q], q, a.cd);
-                    img = gi.y;
-                    if (img >= 0) {
-                        gi = a.fast.images.info[img];
-                        g0 = a.fast.images.nb[2 * (size_t)img];
-                        g1 = a.fast.images.nb[2 * (size_t)img + 1];
-                    }
+                for (int q = 1; q < 27; ++q)
+                    if ((gi.x >> q) & 1)
+                        StoreTraits<S>::bstore(r, slot_offset<S, Off>(gn[post_nb(q)]),
+                                               post_plane(q, FLIP) * LBM3_TILE * int(sizeof(S)), f[q], q, a.cd);
+                img = gi.y;
+                if (img >= 0) {
+                    gi = a.fast.images.info[img];
+                    g0 = a.fast.images.nb[2 * (size_t)img];
+                    g1 = a.fast.images.nb[2 * (size_t)img + 1];
                 }
             }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 27; ++q)
-                StoreTraits<S>::store(at(a.f + post_plane(q, FLIP) * LBM3_TILE, off[post_nb(q)]), f[q], q, a.cd);
         }
     } else {
 #pragma unroll
