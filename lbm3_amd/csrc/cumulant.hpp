@@ -346,7 +346,7 @@ __host__ __device__ __forceinline__ void collide(T (&f)[27], const Relax<T> &R)
 // s, d, k per (x, y) chain along z, 3 (cx + 1) + (cy + 1): h+ + h-, h+ - h-,
 // (h+ + h-) + 4 h0.
 template <int MODE>
-__device__ __forceinline__ void collide_deviations(const float (&s)[9], const float (&d)[9], const float (&k)[9],
+__host__ __device__ __forceinline__ void collide_deviations(const float (&s)[9], const float (&d)[9], const float (&k)[9],
                                                    const float (&U)[3], const Relax<float> &R, float (&h)[27])
 {
     constexpr float n = 1.f / 216.f, third = 1.f / 3.f, ninth = 1.f / 9.f;
