@@ -204,40 +204,43 @@ static bool wide_of(const Sim &s, const Level &l)
 //   sphere 48x24x24 34 -> 18.  FP64: 48x24x24 48 -> 14, 256x128x128 445 -> 328.
 // * the levels in order on one stream: three-level sphere 344, with a stream
 //   per level 384.
-// * wall cells on a side stream again on a refined level of more than 200 MiB,
-//   whose step runs at the copy rate: three states of a three-level sphere in
-//   turn 793 against 822 (finest level 333 MB, 88 cells across) and 619 / 687
-//   (250 MB, 80 across); 385 / 345 at 128 MB (64 across).
 // * block order: one contiguous part per XCD, swept backwards every other step
 //   (order 3), so that each XCD's L2 and the last-level cache still hold what
-//   the step starts on: 64^3 vortex 14.9 against 18.3 in plain order, duct
-//   256x64x64 40 / 44, sphere 256x128x128 (452 MB) 155 / 157.  The plain order
-//   swept backwards (2) wins above about 512 MiB of populations, 300x150x150
-//   (729 MB) 272 against 289, and where rotors make some parts slower than
-//   others: rotor duct 286 / 306.
+//   the step starts on: 64^3 vortex 14.9 against 18.3 in plain order, 118^3 57 /
+//   63, sphere 260x130x130 (453 MiB) 171 / 174.  The plain order swept backwards (2)
+//   wins above about 512 MiB of populations, 272x136x136 (518 MiB) 201 / 203,
+//   300x150x150 272 / 287, FP64 140^3 vortex (590 MiB) 204 / 217, and where rotors
+//   make some parts slower than others: rotor duct 286 / 306.
 // * occupancy cap of the bulk kernel (40 KiB of LDS per block, four blocks per
-//   CU: their tiles then fit an XCD's L2): above 512 MiB, 400x200x200 632
-//   against 692, three 300x150x150 states in turn 302 / 324, one alone the same
-//   within 2%; on the refined levels of more than 200 MiB; and on levels of 64 to 256 MiB without open
-//   cells, three-level sphere 344 / 354, 130^3 vortex 91.2 / 93.2 (50 MB level
-//   25.2 / 23.6, 158^3 vortex of 443 MB 154 / 147).  Never for 16-bit storage,
-//   whose kernels are bound by instructions: FP16 256x128x128 115 / 94,
-//   400x200x200 464 / 380.
+//   CU: their tiles then fit an XCD's L2), each where one simulation alone on the
+//   GPU is faster with it: above 640 MiB, 300x150x150 (695 MiB) 272 against 273,
+//   340x170x170 411 / 418, 400x200x200 659 / 695 (288x144x144 of 615 MiB 237 /
+//   230); on refined levels with walls above 256 MiB, three-level sphere 88 across
+//   (317 MiB) 757 / 767, 100 across 1106 / 1112; and on levels of 64 to 256 MiB
+//   without open cells, 92^3 vortex (86 MiB) 30.4 / 30.8, 118^3 53 / 57, 130^3
+//   (237 MiB) 72 / 91, FP64 104^3 73 / 76 (80^3 of 57 MiB 23.0 / 22.3, 140^3 of 295
+//   MiB 122 / 117).  Several simulations at once on streams of their own want it
+//   earlier: three 272x136x136 in turn 231 / 266.  Never for 16-bit storage,
+//   whose kernels are bound by instructions: FP16 272x136x136 159 / 137,
+//   360x180x180 357 / 285.
+// The levels' wall cells on a side stream, as the three-level sphere above 200
+// MiB had them for several simulations at once (three in turn, 88 across, 833
+// against 894), cost one alone 783 against 757, FP64 64 across 685 against 606.
 Sim::Tune tune_of(const Sim &s, const Level &l)
 {
     if (s.tuneChosen) return s.tune;
     constexpr long long MiB = 1LL << 20;
     const long long size = (long long)storage_bytes(s.storage), bytes = 27 * size * l.N;
     Sim::Tune t;
-    const bool deep = s.levels > 1 && l.W > 0 && !l.openInBulk && l.rotors.empty() && bytes > 200 * MiB;
-    t.overlap = deep ? 1 : 3;
+    t.overlap = 3;
     t.ordered = true;
     // the same on every level: a new layout rebuilds all of them (same_open_layout)
     for (int L = 0; L < s.levels; ++L) t.rotorInBulk |= s.L[L].rotors.empty() ? 0 : 1;
     t.openGroup = 1;
     t.openSplit = s.ownSplit;
     t.xcdRemap = !l.rotors.empty() || bytes > 512 * MiB ? 2 : 3;
-    const bool cap = deep || bytes > 512 * MiB || (!l.openInBulk && bytes > 64 * MiB && bytes <= 256 * MiB);
+    const bool refined = s.levels > 1 && l.W > 0 && l.rotors.empty();
+    const bool cap = bytes > 640 * MiB || (!l.openInBulk && bytes > 64 * MiB && (refined || bytes <= 256 * MiB));
     t.bulkLds = size >= 4 && cap ? LBM3_BULK_LDS : 0;
     return t;
 }
