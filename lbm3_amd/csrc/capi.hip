@@ -1557,8 +1557,11 @@ int lbm3_download_macros(lbm3_sim *h, int level, void *out)
     // allocation and its release, which waits for the device, cost a 32^3 box
     // more than the fields themselves
     const long long bytes = 4LL * l.N * (long long)cb;
+    // (one call at a time; a second thread's waits for it)
+    std::unique_lock<std::mutex> kept(s.keptLock, std::defer_lock);
     DBuf<unsigned char> own;
-    DBuf<unsigned char> &d = bytes <= (64LL << 20) ? s.fields : own;
+    if (bytes <= (64LL << 20)) kept.lock();
+    DBuf<unsigned char> &d = kept.owns_lock() ? s.fields : own;
     if (d.n < bytes) HIPCHK(d.alloc(bytes));
     const bool flip = l.info.esotwistFlipper != 0;
     const Topology t = topo_of(l);
@@ -2359,11 +2362,13 @@ int lbm3_rotor_forces(lbm3_sim *h, int level, int rotor, double *out)
     const int nz = d.nonZero;
     if (nz == 0) return 0;
     const int nb = rotor_force_blocks(nz);
-    if (s.partial.n < 6LL * nb) HIPCHK(s.partial.alloc(6LL * nb));
-    launch_rotor_force(d, R.index.p, s.partial.p, s.stream);
+    // a buffer of its own: another thread may be in a sum that uses `partial`
+    std::lock_guard<std::mutex> kept(s.keptLock);
+    if (s.rotorSums.n < 6LL * nb) HIPCHK(s.rotorSums.alloc(6LL * nb));
+    launch_rotor_force(d, R.index.p, s.rotorSums.p, s.stream);
     HIPCHK(hipGetLastError());
     std::vector<double> host((size_t)nb * 6);
-    HIPCHK(hipMemcpyAsync(host.data(), s.partial.p, sizeof(double) * host.size(), hipMemcpyDeviceToHost, s.stream));
+    HIPCHK(hipMemcpyAsync(host.data(), s.rotorSums.p, sizeof(double) * host.size(), hipMemcpyDeviceToHost, s.stream));
     HIPCHK(hipStreamSynchronize(s.stream));
     for (int b = 0; b < nb; ++b)
         for (int k = 0; k < 6; ++k) out[k] += host[(size_t)b * 6 + k];

@@ -264,10 +264,10 @@ template <class S> struct OpenArgs {
 
 // Dynamic LDS per bulk block, unused by the kernel: a cap on resident bulk
 // blocks per CU (160 KiB / 40 KiB = 4, i.e. 16 of the 32 wave slots a CU has
-// at this kernel's register use).  Measured on the 256x128x128 sphere: the
-// bulk kernel is 1.5% faster than at full occupancy, and the free slots let
-// the wall-adjacent kernel on the second stream run beside it instead of
-// after it (the whole step 7% faster).  The default of Sim::Tune::bulkLds.
+// at this kernel's register use).  Measured on the 256x128x128 sphere with the
+// wall-adjacent kernel on the second stream: the bulk kernel is 1.5% faster than at
+// full occupancy, and the free slots let that kernel run beside it instead of
+// after it (the whole step 7% faster).  tune_of says where one launch gains by it.
 #ifndef LBM3_BULK_LDS
 #define LBM3_BULK_LDS 40960
 #endif

@@ -2,6 +2,7 @@
 #pragma once
 #include <string>
 #include <array>
+#include <mutex>
 #include <vector>
 #include "../../include/lbm3mi.h"
 #include "step.hpp"
@@ -184,7 +185,10 @@ struct Sim {
     std::vector<StepParam> *dryRun = nullptr;
     DBuf<double> partial;            // reduction scratch
     DBuf<double> scalar;
+    // kept between calls, whose threads take turns
+    std::mutex keptLock;
     DBuf<unsigned char> fields;      // lbm3_download_macros, up to 64 MiB
+    DBuf<double> rotorSums;          // lbm3_rotor_forces
     int watchdog = 0;                // lbm3_run checks for non-finite populations every this many coarse steps (0: off)
     std::vector<std::vector<int>> stlEdges;   // shared-edge counts [3 T] of each static body of the last build
     // timing of the level-0 collide-stream launches

@@ -74,8 +74,8 @@ def test_served_matches_single_simulation(name):
     ke = s.kinetic_energy()
     s.close()
     assert res["fluid_updates"] == fu * steps
-    # the server applies the open boundary as its own pass, the single path folds
-    # it into the next step's loads: the same arithmetic, up to contraction
+    # both complete the open boundary at the next load where they can, in kernels
+    # of their own: the same arithmetic, up to contraction
     assert rel_max(m[:, 1:], ref[:, 1:]) < 1e-6
     assert np.max(np.abs(m[:, 0] - ref[:, 0])) < 1e-6
     assert abs(res["kinetic_energy"] / ke - 1.0) < 1e-5
