@@ -28,7 +28,10 @@
 // One object per population storage, compiled side by side (LBM3_STEP_STORE:
 // the LBM3_STORE_* code of this object's storage; undefined: all of them in
 // one object).  What does not depend on the storage is defined in each and
-// merged by the linker; its kernels are local to their object.
+// merged by the linker; its kernels are local to their object.  16-bit storage has
+// a second object (LBM3_STEP_POPULATIONS) with the kernels that collide populations
+// on levels with rotors (launch_bulk, launch_open_groups with DEV false): with them
+// in the first one it took 254 s of the build, the others up to 160.
 #define LBM3_SHARED_DEF __attribute__((weak))
 
 namespace lbm3 {
@@ -1451,7 +1454,7 @@ void launch_collide_wall(const StepArgs<S> &a, bool flip, hipStream_t s)
 
 
 template <class S, bool DEV>
-static void launch_bulk(const StepArgs<S> &a, bool flip, hipStream_t s)
+void launch_bulk(const StepArgs<S> &a, bool flip, hipStream_t s)
 {
     const dim3 g(blocks_for(a.fast.N)), b(256);
     const unsigned lds = (unsigned)a.bulkLds;
@@ -1547,7 +1550,7 @@ void launch_rotor_cells(const StepArgs<S> &a, bool flip, hipStream_t s)
 }
 
 template <class S, int G, bool DEV>
-static void launch_open_groups(const StepArgs<S> &a, bool flip, hipStream_t s)
+void launch_open_groups(const StepArgs<S> &a, bool flip, hipStream_t s)
 {
     const dim3 g((unsigned)((a.open.count + 256 / G - 1) / (256 / G))), b(256);
     const bool k17 = relax_of<typename StoreTraits<S>::compute>(a.bulk).k17 != 0;
@@ -1905,6 +1908,17 @@ LBM3_SHARED_DEF void launch_cut_finish(float *img, long long pixels, const CutUn
 #define LBM3_STEP_STORE -1
 #endif
 #define LBM3_STEP_HAS(store) (LBM3_STEP_STORE == -1 || LBM3_STEP_STORE == store)
+#define LBM3_POPULATION_KERNELS(X, S)                                                        \
+    X template void launch_bulk<S, false>(const StepArgs<S> &, bool, hipStream_t);           \
+    X template void launch_open_groups<S, 8, false>(const StepArgs<S> &, bool, hipStream_t); \
+    X template void launch_open_groups<S, 16, false>(const StepArgs<S> &, bool, hipStream_t);
+#if defined(LBM3_STEP_POPULATIONS)
+#define LBM3_INSTANTIATE_16(S) LBM3_POPULATION_KERNELS(, S)
+#elif LBM3_STEP_STORE == -1
+#define LBM3_INSTANTIATE_16(S) LBM3_INSTANTIATE(S)
+#else
+#define LBM3_INSTANTIATE_16(S) LBM3_POPULATION_KERNELS(extern, S) LBM3_INSTANTIATE(S)
+#endif
 #if LBM3_STEP_HAS(LBM3_STORE_F32)
 LBM3_INSTANTIATE(float)
 template void launch_collide_batch<float>(float *, int, const Relax<float> &, hipStream_t);
@@ -1914,13 +1928,13 @@ LBM3_INSTANTIATE(double)
 template void launch_collide_batch<double>(double *, int, const Relax<double> &, hipStream_t);
 #endif
 #if LBM3_STEP_HAS(LBM3_STORE_F16)
-LBM3_INSTANTIATE(__half)
+LBM3_INSTANTIATE_16(__half)
 #endif
 #if LBM3_STEP_HAS(LBM3_STORE_BF16)
-LBM3_INSTANTIATE(__hip_bfloat16)
+LBM3_INSTANTIATE_16(__hip_bfloat16)
 #endif
 #if LBM3_STEP_HAS(LBM3_STORE_F16C)
-LBM3_INSTANTIATE(f16c)
+LBM3_INSTANTIATE_16(f16c)
 #endif
 
 } // namespace lbm3
