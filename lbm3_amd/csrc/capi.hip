@@ -324,9 +324,14 @@ static int prepare_open_fusion(Sim &s, int L)
     }
     DBuf<int> openOf;
     bool fuse = false;
-    if (L == 0 && l.nOpen > 0) {
+    // without room for the index the open cells keep their pass after streaming
+    bool index = L == 0 && l.nOpen > 0;
+    if (index && openOf.alloc(l.N) != hipSuccess) {
+        (void)hipGetLastError();
+        index = false;
+    }
+    if (index) {
         DBuf<int> flag;
-        HIPCHK(openOf.alloc(l.N));
         HIPCHK(flag.alloc(1));
         HIPCHK(hipMemsetAsync(openOf.p, 0xFF, sizeof(int) * (size_t)l.N, s.stream));
         HIPCHK(hipMemsetAsync(flag.p, 0, sizeof(int), s.stream));
