@@ -1252,8 +1252,8 @@ int lbm3_autotune(lbm3_sim *h, int steps, double *out, int cap, int *nOut)
     const Sim::Tune start = s.tune;
     const bool startChosen = s.tuneChosen;
     // candidate 0: every level's own choices (tune_of), which no single set of
-    // choices gives on several levels: three-level sphere 348 us per step against
-    // 368 for the best single set
+    // choices gives on several levels: three-level sphere 340 us per coarse step
+    // against 368 for the best single set
     struct Cand { Sim::Tune t; bool chosen; double ms; };
     std::vector<Cand> cands;
     auto layout = [&](bool chosen, const Sim::Tune &t) {
